@@ -364,7 +364,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
         const Node<DIM> pj = load_node<DIM>(vrec, NQ, j);
         double Ga[NG];
         for (int c = 0; c < NG; ++c) Ga[c] = hG[r][c] + vrec[(VS + c) * NQ + j];
-        const PairFlux<DIM> P = pair_flux<DIM, false, (R > 1)>(me[r], pj, inv2gm1, smooth_v);
+        const PairFlux<DIM> P = pair_flux<DIM>(me[r], pj, inv2gm1, smooth_v);
         double Dx[DIM];
         for (int d = 0; d < DIM; ++d) Dx[d] = 0.0;
         for (int q = 0; q < DIM; ++q)
@@ -593,7 +593,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
             if (!rv[r]) continue;
             double n[DIM];
             for (int d = 0; d < DIM; ++d) n[d] = a[r][d] + x.b[d];
-            const PairFlux<DIM> P = pair_flux<DIM, false, (R > 1)>(me[r], x.pf, inv2gm1, smooth_f);
+            const PairFlux<DIM> P = pair_flux<DIM>(me[r], x.pf, inv2gm1, smooth_f);
             double Fn[NFLD];
             flux_dot<DIM>(P, n, Fn);
             for (int f = 0; f < NFLD; ++f) {
@@ -799,7 +799,7 @@ surf_kernel(int K, const double *__restrict__ fgeo, const uint32_t *__restrict__
     const double lamM = sqrt(2.0 * a.hq) + sqrt(gamma * pM / UM[0]);
     const double lamP = sqrt(2.0 * b.hq) + sqrt(gamma * pP / UP[0]);
     const double Lfc = ltau * fmax(lamM, lamP) * sJ;
-    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3, (S::R > 1)>(a, b, inv2gm1);
+    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3>(a, b, inv2gm1);
     double Fn[NFLD];
     flux_dot<DIM>(P, nJ, Fn);
     const double *rf = rhsQf + (size_t)k * NFN * NFLD;
@@ -1174,7 +1174,7 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
     const double lamM = sqrt(2.0 * a.hq) + sqrt(gamma * pM / UM[0]);
     const double lamP = sqrt(2.0 * b.hq) + sqrt(gamma * pP / UP[0]);
     const double Lfc = ltau * fmax(lamM, lamP) * sJ;
-    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3, (S::R > 1)>(a, b, inv2gm1);
+    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3>(a, b, inv2gm1);
     double Fn[NFLD];
     flux_dot<DIM>(P, nJ, Fn);
     for (int f = 0; f < NFLD; ++f)

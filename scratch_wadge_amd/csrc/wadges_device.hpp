@@ -40,14 +40,14 @@ template <int DIM> struct Node {
   double hq;       // |u|^2 / 2
 };
 
-// 1/x from v_rcp_f64 refined by two Newton steps (the first half of the compiler's
-// IEEE division sequence, without the final quotient correction): ~1 ulp.
+// 1/x from v_rcp_f64 (relative error below 2^-24 on gfx950, measured over 4M
+// arguments) and one third-order step, r (1 + e + e^2) with e = 1 - x r: the
+// omitted e^3 is below 2^-72.  The same results as two Newton steps (at most half
+// an ulp off on those arguments) in three multiply-adds instead of four.
 __device__ __forceinline__ double rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
 // Conservative state -> node record.  3D multiplies by 1/rho
@@ -103,13 +103,17 @@ template <int DIM> __device__ __forceinline__ double logmean_series2(double u) {
     return 2.0 + u * (2.0 / 3.0 + u * (2.0 / 5.0 + u * (2.0 / 7.0 + u * (2.0 / 9.0))));
 }
 
-// 1 / (2 F(u)) for the 3D series F(u) = 1 + u/3 + u^2/5 + u^3/7, as the
-// series of 1/F to the same order: 1 - u/3 - 4u^2/45 - 44u^3/945 (the
-// coefficients c_n = -sum_k a_k c_{n-k} of the reciprocal of a power series).
-// For u below the series threshold 1e-4 the omitted term is below 1e-17
-// relative, under the rounding of the division it replaces.
-__device__ __forceinline__ double logmean_inv_series2_3d(double u) {
-  return 0.5 + u * (-1.0 / 6.0 + u * (-2.0 / 45.0 + u * (-22.0 / 945.0)));
+// 1 / (2 F(u)) as the series of 1/F to the order of F itself: 1 - u/3 - 4u^2/45
+// - 44u^3/945 (- 428u^4/14175 in 2D) (the coefficients c_n = -sum_k a_k c_{n-k}
+// of the reciprocal of a power series).  Below the series thresholds (u < 1e-4
+// in 3D, 1e-3 in 2D) the omitted term is below 3e-17 relative, under the
+// rounding of the division it replaces.
+template <int DIM> __device__ __forceinline__ double logmean_inv_series2(double u) {
+  if constexpr (DIM == 3)
+    return 0.5 + u * (-1.0 / 6.0 + u * (-2.0 / 45.0 + u * (-22.0 / 945.0)));
+  else
+    return 0.5 +
+           u * (-1.0 / 6.0 + u * (-2.0 / 45.0 + u * (-22.0 / 945.0 + u * (-214.0 / 14175.0))));
 }
 
 // True when p holds on every active lane of the wave (a scalar test).
@@ -138,63 +142,50 @@ __device__ __forceinline__ bool in_smooth_band(double rho, double beta, double r
          fabs(beta - beta_ref) <= kSmoothBand * beta_ref;
 }
 
-// inv2gm1 = 1 / (2 (gamma - 1)).  Lanes of a wave may take different log-mean
-// branches: both are evaluated and selected per lane, with two reciprocals per
-// pair (f of both log means, then the quotients).  In 3D, when every active
-// lane takes the series branch for both log means (smooth states: neighbouring
-// nodes differ by far less than the 1 % that the series threshold allows), a
-// wave-uniform test skips the selection.  With ONE_RCP that path also needs
-// one reciprocal only: 1/(rho_a + rho_b) and 1/(beta_a + beta_b) both come
-// from 1/((rho_a + rho_b)(beta_a + beta_b)), and rho_log = (rho_a + rho_b) /
-// (2 F(u_rho)) uses the series of 1/(2F) instead of a division (equal to
-// round-off); without it the skip gives the same bits as the selection.  The
-// kernels whose register budget has room for the second path's values use
-// ONE_RCP.  (In 2D the kernels aim at four or more waves per SIMD, whose
-// register budget cannot hold both branches' values across the test: it
-// spilled.)
+// inv2gm1 = 1 / (2 (gamma - 1)).  f of both log means and 1/(beta_a + beta_b)
+// come from one reciprocal, 1/((rho_a + rho_b)(beta_a + beta_b)).  The series
+// branch takes rho_log from the series of 1/(2F) and 1/beta_log = 2F/(beta_a +
+// beta_b), so it needs no other; the log branches of both log means share a
+// second reciprocal.  Each lane selects the branch of each log mean by itself, so
+// a pair's bits do not depend on the pairs its wave holds, and every kernel that
+// evaluates a pair gets the same ones.  (Two reciprocals and a selection of both
+// quotients' numerators and denominators, four-term reciprocals: 3D N = 4, K =
+// 13,182, a step 1.79 -> 1.71 ms; 3D N = 3, K = 196,608, 9.05 -> 8.94 ms.)  In 3D, when every active lane takes the
+// series branch of both log means (smooth states: neighbouring nodes differ by far
+// less than the 1 % that the series threshold allows), a wave-uniform test skips
+// the log branches (same bits).  In 2D the test does not pay: the kernels aim at
+// four or more waves per SIMD and spilled with it.
 // smooth: a wave-uniform flag by which the caller guarantees (3D) that every
 // active lane's pair takes the series branch of both log means; the per-pair
 // wave test is then skipped (the same branch, so the same bits).
-template <int DIM, bool LAZY_LOGS = false, bool ONE_RCP = false>
+template <int DIM, bool LAZY_LOGS = false>
 __device__ __forceinline__ PairFlux<DIM> pair_flux(const Node<DIM> &a, const Node<DIM> &b,
                                                    double inv2gm1, bool smooth = false) {
   constexpr double TH = (DIM == 3) ? 1.0e-4 : 1.0e-3;
   const double sr = a.rho + b.rho, dr = a.rho - b.rho;
   const double sb = a.beta + b.beta, db = a.beta - b.beta;
-  // f = (aL-aR)/(aL+aR) for both log means from one reciprocal
   const double q1 = rcp(sr * sb);
-  const double fr = dr * sb * q1;
-  const double fb = db * sr * q1;
+  const double isr = sb * q1, isb = sr * q1;
+  // f = (aL-aR)/(aL+aR) of both log means
+  const double fr = dr * isr, fb = db * isb;
   const double ur = fr * fr, ub = fb * fb;
   const bool serR = ur < TH, serB = ub < TH;
   PairFlux<DIM> P;
-  double ratio;   // rho_log / beta_log
+  P.rholog = sr * logmean_inv_series2<DIM>(ur);
+  double ibl = logmean_series2<DIM>(ub) * isb;   // 1 / beta_log
+  P.pa = 0.5 * sr * isb;
   const bool all_series = DIM == 3 && (smooth || wave_all(serR && serB));
-  if (ONE_RCP && all_series) {
-    const double isb = sr * q1;                       // 1 / sb
-    P.rholog = sr * logmean_inv_series2_3d(ur);
-    P.pa = 0.5 * sr * isb;
-    ratio = P.rholog * logmean_series2<DIM>(ub) * isb;   // beta_log = sb / (2 F(u_beta))
-  } else {
-    const double polyR = logmean_series2<DIM>(ur);
-    const double polyB = logmean_series2<DIM>(ub);
-    // logmean = num / den:  series (aL+aR) / (2 F(u)),  log (aL-aR) / (ln aL - ln aR)
-    double numR = sr, denR = polyR, numB = sb, denB = polyB;
-    if (!all_series) {
-      const double ldR = LAZY_LOGS ? log(a.rho) - log(b.rho) : a.lrho - b.lrho;
-      const double ldB = LAZY_LOGS ? log(a.beta) - log(b.beta) : a.lbeta - b.lbeta;
-      numR = serR ? sr : dr;
-      denR = serR ? polyR : ldR;
-      numB = serB ? sb : db;
-      denB = serB ? polyB : ldB;
-    }
-    // rholog = numR/denR, rholog/betalog = numR denB/(denR numB), pa = (sr/2)/sb
-    const double q = rcp(denR * numB * sb);
-    const double A = numB * q;
-    P.rholog = numR * sb * A;
-    P.pa = 0.5 * sr * denR * A;
-    ratio = numR * denB * sb * q;
+  if (!all_series) {
+    // rho_log = dr / (ln rho_a - ln rho_b), 1/beta_log = (ln beta_a - ln beta_b) / db
+    const double ldR = LAZY_LOGS ? log(a.rho) - log(b.rho) : a.lrho - b.lrho;
+    const double ldB = LAZY_LOGS ? log(a.beta) - log(b.beta) : a.lbeta - b.lbeta;
+    const double dR = serR ? 1.0 : ldR;
+    const double dB = serB ? 1.0 : db;
+    const double q2 = rcp(dR * dB);
+    P.rholog = serR ? P.rholog : dr * dB * q2;
+    ibl = serB ? ibl : ldB * dR * q2;
   }
+  const double ratio = P.rholog * ibl;           // rho_log / beta_log
   double vv = 0.0;
   for (int d = 0; d < DIM; ++d) {
     P.va[d] = a.hv[d] + b.hv[d];
@@ -358,7 +349,7 @@ __device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DI
       // l' = 2 f F'(u) / (s F^2)  (the partials of the series branch)
       auto partials = [&](double sa, double is, double f, double u, double x, double y,
                           double &l, double &dx, double &dy, double &i2F) {
-        const double h = logmean_inv_series2_3d(u);          // 1/(2F)
+        const double h = logmean_inv_series2<DIM>(u);          // 1/(2F)
         const double Fp = 1.0 / 3.0 + u * (2.0 / 5.0 + u * (3.0 / 7.0));
         l = sa * h;
         const double t = 8.0 * f * Fp * is * h * h;           // 2 f F' / (s F^2)
