@@ -223,14 +223,13 @@ template <class S> struct VolSmem {
   static_assert(per_elem >= 2 * acc_v, "the fused stage's update needs two [NFLD][NQ] buffers");
 };
 
-// Waves per SIMD that the LDS of a one-wave workgroup of `bytes` allows (160 KiB
-// of LDS per CU, four SIMDs), rounded up.  Kernels whose occupancy LDS limits
+// Waves per SIMD that the LDS of a one-wave workgroup of `bytes` allows on every
+// SIMD (160 KiB of LDS per CU, four SIMDs).  Kernels whose occupancy LDS limits
 // declare it, so that the compiler may spend the registers that occupancy
 // leaves free on latency hiding (batched loads, unrolled row products) instead
 // of aiming at an occupancy the LDS cannot reach.
 constexpr int lds_waves_per_simd(int bytes) {
-  const int wg = (160 * 1024) / (bytes > 0 ? bytes : 1);
-  const int w = (wg + 3) / 4;
+  const int w = (160 * 1024) / (bytes > 0 ? bytes : 1) / 4;
   return w < 1 ? 1 : (w > 8 ? 8 : w);
 }
 
@@ -295,14 +294,16 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
   bool rv[R];                               // row r of this lane exists
   for (int r = 0; r < R; ++r) rv[r] = valid && (r == 0 || l + r * LPE < NQ);
 
-  // Smooth waves (3D): every node of the wave's elements within a band of
-  // element 0's node 0 (read from LDS) in rho and beta; the loops then skip the
-  // per-pair branch test of the log means, and the face records take their
-  // logarithms only when a wave is not smooth (same bits).  Taken where it
-  // pays: with two rows per lane (3D N = 3: 1.6 % and 2.2 % faster on the
-  // Taylor-Green state); at 3D N = 4 the test measured 1.5 % slower.
+  // Smooth waves: every node of the wave's elements within a band of element 0's
+  // node 0 (read from LDS) in rho and beta.  The face records, in 2D the volume
+  // records too, then go without their logarithms (two of 50 instructions per node;
+  // almost every wave of the Taylor-Green state, 93 % of the vortex ensemble's), and
+  // with two rows per lane (3D N = 3) the loops skip the per-pair branch test of the
+  // log means (same bits).  With one row per lane the 3D kernels have no registers
+  // for it (spills; skipping the test at N = 4 measured 1.5 % slower).
   constexpr bool SMOOTH_LOOPS = DIM == 3 && R > 1;
-  constexpr bool LAZY = SMOOTH_LOOPS;   // face-record logarithms only where needed
+  constexpr bool LAZY = DIM == 2 || R > 1;   // face records
+  constexpr bool LAZY_V = DIM == 2;          // volume records
 
   // ---------------- phase 1: volume records, volume-volume block
   Node<DIM> me[R];
@@ -312,7 +313,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
     const int i = l + r * LPE;
     double U[NFLD];
     for (int f = 0; f < NFLD; ++f) U[f] = Uq[i + f * NQ];
-    me[r] = make_node<DIM>(U, gm1);
+    me[r] = make_node<DIM, !LAZY_V>(U, gm1);
     for (int c = 0; c < NG; ++c) hG[r][c] = 0.5 * vg[i + c * NQ];
     store_node<DIM>(vrec, NQ, i, me[r]);
     for (int c = 0; c < NG; ++c) vrec[(VS + c) * NQ + i] = hG[r][c];
@@ -322,12 +323,20 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
 
   const double rho_ref = wc.smem[NFLD * NQ];
   const double beta_ref = wc.smem[NFLD * NQ + (DIM + 1) * NQ];
-  bool smooth_v = false;
-  if constexpr (SMOOTH_LOOPS) {
-    bool ok = true;
-    for (int r = 0; r < R; ++r)
-      if (rv[r]) ok = ok && in_smooth_band(me[r].rho, me[r].beta, rho_ref, beta_ref);
-    smooth_v = uniform_flag(wave_all(ok));
+  bool in_band = LAZY;
+  for (int r = 0; r < R; ++r)
+    if (LAZY && rv[r]) in_band = in_band && in_smooth_band<DIM>(me[r].rho, me[r].beta, rho_ref, beta_ref);
+  const bool smooth_v = uniform_flag(wave_all(in_band));
+  if (LAZY_V && !smooth_v) {
+    // the log branch may be taken: logarithms of the volume records
+    for (int r = 0; r < R; ++r) {
+      if (!rv[r]) continue;
+      me[r].lrho = ln(me[r].rho);
+      me[r].lbeta = ln(me[r].beta);
+      vrec[(DIM + 2) * NQ + l + r * LPE] = me[r].lrho;
+      vrec[(DIM + 3) * NQ + l + r * LPE] = me[r].lbeta;
+    }
+    __syncthreads();
   }
 
   for (int r = 0; r < R; ++r)
@@ -335,7 +344,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
 
   // 3D N = 2 (Nq = 11): its short loops (6 steps here and in the face walk) are
   // kept rolled; unrolled completely they spill even at 168 registers.
-  constexpr bool ROLLED = S::DIM == 3 && NQ == 11;
+  constexpr bool ROLLED = (S::DIM == 3 && NQ == 11) || (S::DIM == 2 && NQ <= 6);
   int vv_steps = TVT;
   if constexpr (ROLLED) vv_steps = opaque_bound(TVT);
   if (valid) {
@@ -364,7 +373,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
         const Node<DIM> pj = load_node<DIM>(vrec, NQ, j);
         double Ga[NG];
         for (int c = 0; c < NG; ++c) Ga[c] = hG[r][c] + vrec[(VS + c) * NQ + j];
-        const PairFlux<DIM> P = pair_flux<DIM>(me[r], pj, inv2gm1, smooth_v);
+        const PairFlux<DIM> P = pair_flux<DIM>(me[r], pj, inv2gm1, SMOOTH_LOOPS && smooth_v);
         double Dx[DIM];
         for (int d = 0; d < DIM; ++d) Dx[d] = 0.0;
         for (int q = 0; q < DIM; ++q)
@@ -385,7 +394,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
       if constexpr (PIPE) {
         double nDf[R][DIM], nDb[R][DIM];
         fetch(0, nDf, nDb);
-        for (int t = 0; t < TVT; ++t) {
+        for (int t = 0; t < vv_steps; ++t) {
           if (2 * t > NQ) break;
           double Df[R][DIM], Db[R][DIM];
           for (int r = 0; r < R; ++r)
@@ -530,7 +539,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
       double U[NFLD];
       for (int f = 0; f < NFLD; ++f) U[f] = Uft[fn + f * NFN];
       const Node<DIM> nf = make_node<DIM, !LAZY>(U, gm1);
-      if constexpr (SMOOTH_LOOPS) ok_f = ok_f && in_smooth_band(nf.rho, nf.beta, rho_ref, beta_ref);
+      ok_f = ok_f && in_smooth_band<DIM>(nf.rho, nf.beta, rho_ref, beta_ref);
       store_node<DIM>(frect, NH, fl, nf);
       const int face = fn / NFQ;
       for (int d = 0; d < DIM; ++d) {
@@ -540,16 +549,24 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
       }
     }
     __syncthreads();
-    const bool smooth_f = SMOOTH_LOOPS && uniform_flag(smooth_v && wave_all(ok_f));
-    if (LAZY && !smooth_f) {
-      // the log branch may be taken: logarithms of this part's face records
+    const bool smooth_w = uniform_flag(smooth_v && wave_all(ok_f));
+    const bool smooth_f = SMOOTH_LOOPS && smooth_w;
+    if (LAZY && !smooth_w) {
+      // the log branch may be taken: logarithms of this part's face records, and
+      // of the lane's rows where the volume block went without
+      if (LAZY_V && smooth_v)
+        for (int r = 0; r < R; ++r) {
+          if (!rv[r]) continue;
+          me[r].lrho = ln(me[r].rho);
+          me[r].lbeta = ln(me[r].beta);
+        }
       for (int p = wc.lane; p < TPW * NH; p += WAVE) {
         const int t = p / NH;
         const int fl = p - t * NH;
         if (wc.kfirst + t >= wc.K) continue;
         double *frect = wc.smem + t * PER + NFLD * NQ;
-        frect[(DIM + 2) * NH + fl] = log(frect[0 * NH + fl]);
-        frect[(DIM + 3) * NH + fl] = log(frect[(DIM + 1) * NH + fl]);
+        frect[(DIM + 2) * NH + fl] = ln(frect[0 * NH + fl]);
+        frect[(DIM + 3) * NH + fl] = ln(frect[(DIM + 1) * NH + fl]);
       }
       __syncthreads();
     }
@@ -790,16 +807,11 @@ surf_kernel(int K, const double *__restrict__ fgeo, const uint32_t *__restrict__
     double nJ[DIM];
     for (int d = 0; d < DIM; ++d) nJ[d] = g[fn + d * NFN];
     const double sJ = g[fn + DIM * NFN];
-    // 3D: the logarithms are taken only if a lane of the wave needs the log branch
-    const Node<DIM> a = make_node<DIM, DIM == 2>(UM, gm1);
-    const Node<DIM> b = make_node<DIM, DIM == 2>(UP, gm1);
-    // wave speed |u| + sqrt(gamma p / rho)  (okl/Euler3D.okl:3316-3321); 2 hq = |u|^2 exactly
-    const double pM = gm1 * (UM[NFLD - 1] - 0.5 * UM[0] * (2.0 * a.hq));
-    const double pP = gm1 * (UP[NFLD - 1] - 0.5 * UP[0] * (2.0 * b.hq));
-    const double lamM = sqrt(2.0 * a.hq) + sqrt(gamma * pM / UM[0]);
-    const double lamP = sqrt(2.0 * b.hq) + sqrt(gamma * pP / UP[0]);
-    const double Lfc = ltau * fmax(lamM, lamP) * sJ;
-    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3>(a, b, inv2gm1);
+    // the logarithms are taken only if a lane of the wave needs the log branch
+    const Node<DIM> a = make_node<DIM, false>(UM, gm1);
+    const Node<DIM> b = make_node<DIM, false>(UP, gm1);
+    const double Lfc = ltau * fmax(node_speed<DIM>(a, gamma), node_speed<DIM>(b, gamma)) * sJ;
+    const PairFlux<DIM> P = pair_flux<DIM, true>(a, b, inv2gm1);
     double Fn[NFLD];
     flux_dot<DIM>(P, nJ, Fn);
     const double *rf = rhsQf + (size_t)k * NFN * NFLD;
@@ -966,7 +978,7 @@ update_kernel(int K, const double *__restrict__ Jq, const double *__restrict__ V
     J[x] = invJ[x] = 1.0;
     if (rv[x]) {
       J[x] = Jq[(size_t)k * NQ + ir[x]];
-      invJ[x] = 1.0 / J[x];
+      invJ[x] = rcp(J[x]);
       for (int f = 0; f < NFLD; ++f) bufA[e][f][ir[x]] = rhsQ[base + ir[x] + f * NQ];
     }
   }
@@ -979,7 +991,7 @@ update_kernel(int K, const double *__restrict__ Jq, const double *__restrict__ V
       for (int x = 0; x < R; ++x)
         if (rv[x])
           for (int f = 0; f < NFLD; ++f)
-            bufB[e][f][ir[x]] = (DIM == 3) ? r[x][f] * invJ[x] : r[x][f] / J[x];
+            bufB[e][f][ir[x]] = (DIM == 3) ? r[x][f] * invJ[x] : quot(r[x][f], J[x], invJ[x]);
   }
   __syncthreads();
   // r = VqPq bufB ; RK update ; bufA = v(Q) J
@@ -1010,7 +1022,7 @@ update_kernel(int K, const double *__restrict__ Jq, const double *__restrict__ V
       for (int x = 0; x < R; ++x)
         if (rv[x])
           for (int f = 0; f < NFLD; ++f)
-            bufB[e][f][ir[x]] = (DIM == 3) ? r[x][f] * invJ[x] : r[x][f] / J[x];
+            bufB[e][f][ir[x]] = (DIM == 3) ? r[x][f] * invJ[x] : quot(r[x][f], J[x], invJ[x]);
   }
   __syncthreads();
   // bufA = VqPq bufB   (entropy variables v~: the product leaves them in bufA)
@@ -1125,18 +1137,21 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
   vol_body<S>(valid, l, A->rhsQ_in + base, A->vgeo + kk * NQ * NG, s_nref, A->ws, accV, gm1,
               inv2gm1, acc, wc);
 
-  // The update's per-row inputs.  With R > 1 and in 2D they are loaded now, so
-  // that their HBM latency passes under the surface and lift phases (2D: the
-  // ensemble 3 % and the single-problem stage 4 % faster).  The 3D one-row
-  // shapes load them where they are used: N = 2 has no registers to spare, and
-  // at N = 4 loading them early measured the same.
-  constexpr bool EARLY = R > 1 || DIM == 2;
+  // The update's per-row inputs.  With R > 1 and in 2D from N = 3 on they are
+  // loaded now, so that their HBM latency passes under the surface and lift phases
+  // (2D: the ensemble 3 % and the single-problem stage 4 % faster).  2D N = 1 and 2
+  // have no registers for them during the surface flux and load them after it; the
+  // 3D one-row shapes load them where they are used: N = 2 has no registers to
+  // spare, and at N = 4 loading them early measured the same.
+  constexpr bool EARLY = R > 1 || (DIM == 2 && NQ >= 12);
+  constexpr bool HELD = R > 1 || DIM == 2;
   int ir[R];
   for (int r = 0; r < R; ++r) ir[r] = rv[r] ? l + r * LPE : 0;
-  double Qin[EARLY ? R : 1][NFLD], resin[EARLY ? R : 1][NFLD], J[R];
-  for (int r = 0; r < R; ++r) {
-    J[r] = 1.0;
-    if (EARLY && rv[r]) {
+  double Qin[HELD ? R : 1][NFLD], resin[HELD ? R : 1][NFLD], J[R];
+  auto load_rows = [&]() {
+    for (int r = 0; r < R; ++r) {
+      J[r] = 1.0;
+      if (!rv[r]) continue;
       J[r] = A->Jq[kk * NQ + ir[r]];
       for (int f = 0; f < NFLD; ++f) {
         const size_t id = base + ir[r] + f * NQ;
@@ -1144,10 +1159,12 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
         resin[r][f] = A->resQ_in[id];
       }
     }
-  }
+  };
+  if constexpr (EARLY) load_rows();
 
   // ---------------- surface flux + LF penalty, in place over the face rows.
   // The face points of all TPW elements are spread over the whole wave.
+#pragma unroll 1
   for (int p = lane; p < TPW * NFN; p += WAVE) {
     const int t = p / NFN;
     const int fn = p - t * NFN;
@@ -1166,20 +1183,17 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
     double nJ[DIM];
     for (int d = 0; d < DIM; ++d) nJ[d] = g[fn + d * NFN];
     const double sJ = g[fn + DIM * NFN];
-    // 3D: the logarithms are taken only if a lane of the wave needs the log branch
-    const Node<DIM> a = make_node<DIM, DIM == 2>(UM, gm1);
-    const Node<DIM> b = make_node<DIM, DIM == 2>(UP, gm1);
-    const double pM = gm1 * (UM[NFLD - 1] - 0.5 * UM[0] * (2.0 * a.hq));
-    const double pP = gm1 * (UP[NFLD - 1] - 0.5 * UP[0] * (2.0 * b.hq));
-    const double lamM = sqrt(2.0 * a.hq) + sqrt(gamma * pM / UM[0]);
-    const double lamP = sqrt(2.0 * b.hq) + sqrt(gamma * pP / UP[0]);
-    const double Lfc = ltau * fmax(lamM, lamP) * sJ;
-    const PairFlux<DIM> P = pair_flux<DIM, DIM == 3>(a, b, inv2gm1);
+    // the logarithms are taken only if a lane of the wave needs the log branch
+    const Node<DIM> a = make_node<DIM, false>(UM, gm1);
+    const Node<DIM> b = make_node<DIM, false>(UP, gm1);
+    const double Lfc = ltau * fmax(node_speed<DIM>(a, gamma), node_speed<DIM>(b, gamma)) * sJ;
+    const PairFlux<DIM> P = pair_flux<DIM, true>(a, b, inv2gm1);
     double Fn[NFLD];
     flux_dot<DIM>(P, nJ, Fn);
     for (int f = 0; f < NFLD; ++f)
       accFt[f * NFN + fn] = 0.5 * Fn[f] + accFt[f * NFN + fn] - Lfc * (UP[f] - UM[f]);
   }
+  if constexpr (HELD && !EARLY) load_rows();
   __syncthreads();
   // ---------------- RHS rows = volume part + lift of the face terms
   const int nvalid = A->K - kfirst < TPW ? A->K - kfirst : TPW;   // elements of this wave
@@ -1202,9 +1216,10 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
   double invJ[R];
   for (int r = 0; r < R; ++r) {
     invJ[r] = 1.0;
+    if (!HELD) J[r] = 1.0;
     if (rv[r]) {
-      if (!EARLY) J[r] = A->Jq[kk * NQ + ir[r]];
-      invJ[r] = 1.0 / J[r];
+      if (!HELD) J[r] = A->Jq[kk * NQ + ir[r]];
+      invJ[r] = rcp(J[r]);
       for (int f = 0; f < NFLD; ++f) bufA[f * NQ + ir[r]] = rhs[r][f];
     }
   }
@@ -1228,7 +1243,7 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
       for (int r = 0; r < R; ++r) {
         if (!rv[r]) continue;
         for (int f = 0; f < NFLD; ++f)
-          bufB[f * NQ + ir[r]] = (DIM == 3) ? res[r][f] * invJ[r] : res[r][f] / J[r];
+          bufB[f * NQ + ir[r]] = (DIM == 3) ? res[r][f] * invJ[r] : quot(res[r][f], J[r], invJ[r]);
       }
   }
   __syncthreads();
@@ -1241,9 +1256,9 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
         double U[NFLD], V[NFLD];
         for (int f = 0; f < NFLD; ++f) {
           const size_t id = base + ir[r] + f * NQ;
-          const double rq = fa * (EARLY ? resin[r][f] : A->resQ_in[id]) + fdt * res[r][f];
+          const double rq = fa * (HELD ? resin[r][f] : A->resQ_in[id]) + fdt * res[r][f];
           A->resQ[id] = rq;
-          U[f] = (EARLY ? Qin[r][f] : A->Q_in[id]) + fb * rq;
+          U[f] = (HELD ? Qin[r][f] : A->Q_in[id]) + fb * rq;
           A->Q[id] = U[f];
         }
         entropy_vars<DIM>(U, gamma, V);
@@ -1258,7 +1273,7 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
       for (int r = 0; r < R; ++r) {
         if (!rv[r]) continue;
         for (int f = 0; f < NFLD; ++f)
-          bufB[f * NQ + ir[r]] = (DIM == 3) ? res[r][f] * invJ[r] : res[r][f] / J[r];
+          bufB[f * NQ + ir[r]] = (DIM == 3) ? res[r][f] * invJ[r] : quot(res[r][f], J[r], invJ[r]);
       }
   }
   __syncthreads();
@@ -1271,6 +1286,7 @@ __device__ __forceinline__ void stage_body(const ConstArgs *A, double fa, double
   constexpr int WOFF = 2 * NFLD * NQ;
   stage_product_mfma<S, NFN, NQ, NFN, NQ, NFN>(A->VfPq, 0, WOFF, smem, lane, nvalid);
   __syncthreads();
+#pragma unroll 1
   for (int p = lane; p < TPW * NFN; p += WAVE) {
     const int t = p / NFN;
     const int fn = p - t * NFN;
@@ -1323,8 +1339,9 @@ diag_kernel(int K, const double *__restrict__ wq, const double *__restrict__ Jq,
     const double wJ = wq[i] * Jq[(size_t)k * NQ + i];
     double mm = U[1] * U[1];
     for (int d = 1; d < DIM; ++d) mm = mm + U[1 + d] * U[1 + d];
-    const double rhoe = U[NFLD - 1] - 0.5 * mm / U[0];
-    const double s = log((gamma - 1.0) * rhoe) - gamma * log(U[0]);
+    const double irho = rcp(U[0]);
+    const double rhoe = U[NFLD - 1] - quot(0.5 * mm, U[0], irho);
+    const double s = ln((gamma - 1.0) * rhoe) - gamma * ln(U[0]);
     double err = 0.0;
     if (Qex) {
       for (int f = 0; f < NFLD; ++f) {
@@ -1332,7 +1349,7 @@ diag_kernel(int K, const double *__restrict__ wq, const double *__restrict__ Jq,
         err = err + e * e;
       }
     }
-    part[team][0][i] = 0.5 * mm / U[0] * wJ;
+    part[team][0][i] = quot(0.5 * mm, U[0], irho) * wJ;
     part[team][1][i] = wJ * (-U[0] * s);
     part[team][2][i] = err * wJ;
     part[team][3][i] = wJ * U[0];

@@ -414,7 +414,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
   double U[NFLD], J = 1.0, invJ = 1.0;
   if (valid) {
     J = Jq[(size_t)k * NQ + i];
-    invJ = 1.0 / J;
+    invJ = rcp(J);
     for (int f = 0; f < NFLD; ++f) U[f] = Q[base + i + f * NQ];
     double V[NFLD];
     entropy_vars<DIM>(U, gamma, V);
@@ -453,6 +453,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
     if (kt >= K) continue;
     double V[NFLD], Ub[NFLD], g[NFLD];
     for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
+#pragma unroll 4
     for (int j = 0; j < NQ; ++j) {
       const double P = Pf(fn + j * NFN);
       for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[et][f][j];
@@ -466,6 +467,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
   if (valid) {
     double r[NFLD];
     for (int f = 0; f < NFLD; ++f) r[f] = bufB[e][f][i];
+#pragma unroll 8
     for (int fn = 0; fn < NFN; ++fn) {
       const double P = Pf(fn + i * NFN);
       for (int f = 0; f < NFLD; ++f) r[f] += P * bufF[e][f][fn];

@@ -50,6 +50,111 @@ __device__ __forceinline__ double rcp(double x) {
   return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
+// a/b given r = rcp(b): one correction of the quotient by its remainder (within
+// 0.51 ulp for normal operands) instead of the scaled IEEE sequence.
+__device__ __forceinline__ double quot(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
+
+// Logarithm, exponential and square root are evaluated once or more per node; the
+// math library's take 98, 42 and 22 vector instructions in FP64, and its logarithm
+// alone was a fifth of the 2D stage's.  The three below take 50, 27 and 15 and are as
+// accurate: against 80-bit arithmetic over 4M arguments each, rms error ln 0.289
+// ulp (library 0.289-0.293; arguments in [1/2, 2], [1e-6, 1e6], [1e-300, 1e300]),
+// expo 0.302 (0.302; [-8, 8], [-700, 700]), root 0.289 (0.289).  Arguments outside
+// their domain give what the library gives (NaN, infinities, zero).  With them and
+// quot() in place of IEEE division: 2D N = 4, K = 32,258, a step 434 -> 397 us; the
+// 64-problem ensemble 3.11 -> 2.83 ms for two steps; 3D N = 3, K = 196,608, 8.9 ->
+// 8.75 ms.
+
+// A constant in a scalar register at its use.  As plain literals the compiler
+// keeps the coefficients of ln in vector registers across the kernel (20-40
+// registers, spills in the stage kernels).
+__device__ __forceinline__ double sconst(double v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+constexpr double LN2_HI = 0x1.62e42fefp-1;           // 32 bits: k LN2_HI is exact, |k| < 2^20
+constexpr double LN2_LO = 0x1.473de6af278edp-34;     // ln 2 - LN2_HI
+
+// ln x: x = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact), s = f/(2+f)
+// and ln(1+f) = 2 atanh(s) = f - f^2/2 + s (f^2/2 + R(s^2)) with R(z) = 2 (z/3 +
+// z^2/5 + ...) (s f = f^2/2 - s f^2/2 ... regroups the first term so that f enters
+// exactly); the series to z^10, whose omitted term is below 2e-19.  k ln 2, f and
+// f^2/2 are added with their rounding errors.
+__device__ __forceinline__ double ln(double x) {
+  double m = __builtin_amdgcn_frexp_mant(x);                 // [1/2, 1)
+  const int low = m < sconst(0x1.6a09e667f3bcdp-1) ? 1 : 0;
+  m = __builtin_amdgcn_ldexp(m, low);
+  const double k = (double)(__builtin_amdgcn_frexp_exp(x) - low);
+  const double f = m - 1.0;
+  const double s = f * rcp(2.0 + f);
+  const double z = s * s, w = z * z;
+  double r1 = sconst(2.0 / 19.0), r2 = sconst(2.0 / 21.0);
+  r1 = __builtin_fma(w, r1, sconst(2.0 / 15.0));
+  r2 = __builtin_fma(w, r2, sconst(2.0 / 17.0));
+  r1 = __builtin_fma(w, r1, sconst(2.0 / 11.0));
+  r2 = __builtin_fma(w, r2, sconst(2.0 / 13.0));
+  r1 = __builtin_fma(w, r1, sconst(2.0 / 7.0));
+  r2 = __builtin_fma(w, r2, sconst(2.0 / 9.0));
+  r1 = __builtin_fma(w, r1, sconst(2.0 / 3.0));
+  r2 = __builtin_fma(w, r2, sconst(2.0 / 5.0));
+  const double hf = 0.5 * f;
+  const double q = hf * f;
+  const double q_lo = __builtin_fma(hf, f, -q);
+  const double t = s * (q + z * (r1 + z * r2));
+  const double a = k * sconst(LN2_HI);
+  const double b = a + f;                                    // |a| > |f| or a = 0
+  const double b_lo = f - (b - a);
+  const double c = b - q;
+  const double c_lo = (b - c) - q;
+  const double lo = __builtin_fma(k, sconst(LN2_LO), t - q_lo) + (b_lo + c_lo);
+  const double v = c + lo;
+  // 0, negative, infinite and NaN arguments: as the single-precision instruction
+  return __builtin_amdgcn_class(x, 0x180) ? v : (double)__builtin_amdgcn_logf((float)x);
+}
+
+// exp x = 2^n exp(r), r = x - n ln 2 in [-ln 2 / 2, ln 2 / 2], Taylor series to
+// r^13 (the omitted term is below 5e-18).
+__device__ __forceinline__ double expo(double x) {
+  const double n = __builtin_rint(x * sconst(1.4426950408889634));
+  const double r = __builtin_fma(-n, sconst(LN2_LO), __builtin_fma(-n, sconst(LN2_HI), x));
+  double p = sconst(1.0 / 6227020800.0);
+  p = __builtin_fma(p, r, sconst(1.0 / 479001600.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 39916800.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 3628800.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 362880.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 40320.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 5040.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 720.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 120.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 24.0));
+  p = __builtin_fma(p, r, sconst(1.0 / 6.0));
+  p = __builtin_fma(p, r, 0.5);
+  p = __builtin_fma(p, r, 1.0);
+  p = __builtin_fma(p, r, 1.0);
+  double v = __builtin_amdgcn_ldexp(p, (int)n);
+  v = x > sconst(710.0) ? __builtin_huge_val() : v;
+  return x < sconst(-746.0) ? 0.0 : v;
+}
+
+// 1/sqrt(x) for x > 0: v_rsq_f64 and one third-order step.
+__device__ __forceinline__ double rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+// sqrt(x) from it, corrected by the remainder x - s^2.
+__device__ __forceinline__ double root(double x) {
+  const double y = rsqrt_pos(x);
+  const double s = x * y;
+  const double v = __builtin_fma(__builtin_fma(-s, s, x), 0.5 * y, s);
+  return __builtin_amdgcn_class(x, 0x260) ? x : v;           // +-0, +inf
+}
+
 // Conservative state -> node record.  3D multiplies by 1/rho
 // (okl/Euler3D.okl:2252-2256, TESTING); 2D divides (okl/Euler2D.okl:1127-1129).
 // LOGS = false leaves ln rho and ln beta out, for a node that serves a single
@@ -61,21 +166,19 @@ __device__ __forceinline__ Node<DIM> make_node(const double (&U)[DIM + 2], doubl
   n.rho = U[0];
   double v[DIM];
   if constexpr (DIM == 3) {
-    const double inv = 1.0 / U[0];
+    const double inv = rcp(U[0]);
     for (int d = 0; d < DIM; ++d) v[d] = U[1 + d] * inv;
   } else {
-    for (int d = 0; d < DIM; ++d) v[d] = U[1 + d] / U[0];
+    const double inv = rcp(U[0]);
+    for (int d = 0; d < DIM; ++d) v[d] = quot(U[1 + d], U[0], inv);
   }
   double uu = v[0] * v[0];
   for (int d = 1; d < DIM; ++d) uu = uu + v[d] * v[d];
   const double p = gm1 * (U[DIM + 1] - 0.5 * U[0] * uu);
-  if constexpr (DIM == 3)
-    n.beta = U[0] / (2.0 * p);
-  else
-    n.beta = 0.5 * U[0] / p;
+  n.beta = quot(0.5 * U[0], p, rcp(p));
   for (int d = 0; d < DIM; ++d) n.hv[d] = 0.5 * v[d];
-  n.lrho = LOGS ? log(n.rho) : 0.0;
-  n.lbeta = LOGS ? log(n.beta) : 0.0;
+  n.lrho = LOGS ? ln(n.rho) : 0.0;
+  n.lbeta = LOGS ? ln(n.beta) : 0.0;
   n.hq = 0.5 * uu;
   return n;
 }
@@ -128,18 +231,21 @@ __device__ __forceinline__ bool uniform_flag(bool p) {
   return __builtin_amdgcn_readfirstlane((int)p) != 0;
 }
 
-// Smooth waves (3D).  A node is in band when its rho and beta lie within a
-// relative kSmoothBand of a reference node's.  When every node of a wave's
-// elements is in band, every pair (a, b) of them has |a - b| / (a + b) <=
-// band / (1 - band) < 0.0099, so f^2 < 1e-4: both log means of every pair take
-// the 3D series branch, and the pair routines may skip their per-pair wave test
+// Smooth waves.  A node is in band when its rho and beta lie within a relative
+// SmoothBand of a reference node's.  When every node of a wave's elements is in
+// band, every pair (a, b) of them has |a - b| / (a + b) <= band / (1 - band), so f^2
+// < 9.8e-5 (3D) or 9.97e-4 (2D), below the series thresholds: both log means of
+// every pair take the series branch.  The records' logarithms are then never
+// used and not taken (2D N = 4, K = 32,258, a step 397 -> 376 us; 2D N = 3, K =
+// 51,200, 434 -> 405 us), and the pair routines may skip their per-pair wave test
 // (the branch they take is the same, so are the bits).
-constexpr double kSmoothBand = 0.0098;
+template <int DIM> constexpr double smooth_band() { return DIM == 3 ? 0.0098 : 0.0306; }
 
+template <int DIM>
 __device__ __forceinline__ bool in_smooth_band(double rho, double beta, double rho_ref,
                                                double beta_ref) {
-  return fabs(rho - rho_ref) <= kSmoothBand * rho_ref &&
-         fabs(beta - beta_ref) <= kSmoothBand * beta_ref;
+  return fabs(rho - rho_ref) <= smooth_band<DIM>() * rho_ref &&
+         fabs(beta - beta_ref) <= smooth_band<DIM>() * beta_ref;
 }
 
 // inv2gm1 = 1 / (2 (gamma - 1)).  f of both log means and 1/(beta_a + beta_b)
@@ -153,8 +259,10 @@ __device__ __forceinline__ bool in_smooth_band(double rho, double beta, double r
 // 13,182, a step 1.79 -> 1.71 ms; 3D N = 3, K = 196,608, 9.05 -> 8.94 ms.)  In 3D, when every active lane takes the
 // series branch of both log means (smooth states: neighbouring nodes differ by far
 // less than the 1 % that the series threshold allows), a wave-uniform test skips
-// the log branches (same bits).  In 2D the test does not pay: the kernels aim at
-// four or more waves per SIMD and spilled with it.
+// the log branches (same bits).  In the 2D pair loops the test does not pay: the
+// kernels aim at four or more waves per SIMD and spilled with it.  LAZY_LOGS: the
+// nodes come without logarithms, which are taken only behind that test (the
+// surface flux, whose two nodes serve one pair).
 // smooth: a wave-uniform flag by which the caller guarantees (3D) that every
 // active lane's pair takes the series branch of both log means; the per-pair
 // wave test is then skipped (the same branch, so the same bits).
@@ -174,11 +282,11 @@ __device__ __forceinline__ PairFlux<DIM> pair_flux(const Node<DIM> &a, const Nod
   P.rholog = sr * logmean_inv_series2<DIM>(ur);
   double ibl = logmean_series2<DIM>(ub) * isb;   // 1 / beta_log
   P.pa = 0.5 * sr * isb;
-  const bool all_series = DIM == 3 && (smooth || wave_all(serR && serB));
+  const bool all_series = (DIM == 3 || LAZY_LOGS) && (smooth || wave_all(serR && serB));
   if (!all_series) {
     // rho_log = dr / (ln rho_a - ln rho_b), 1/beta_log = (ln beta_a - ln beta_b) / db
-    const double ldR = LAZY_LOGS ? log(a.rho) - log(b.rho) : a.lrho - b.lrho;
-    const double ldB = LAZY_LOGS ? log(a.beta) - log(b.beta) : a.lbeta - b.lbeta;
+    const double ldR = LAZY_LOGS ? ln(a.rho * rcp(b.rho)) : a.lrho - b.lrho;
+    const double ldB = LAZY_LOGS ? ln(a.beta * rcp(b.beta)) : a.lbeta - b.lbeta;
     const double dR = serR ? 1.0 : ldR;
     const double dB = serB ? 1.0 : db;
     const double q2 = rcp(dR * dB);
@@ -208,6 +316,13 @@ __device__ __forceinline__ void flux_dot(const PairFlux<DIM> &P, const double (&
   out[DIM + 1] = P.f4aux * Un;
 }
 
+// Wave speed |u| + sqrt(gamma p / rho) of a node (okl/Euler3D.okl:3316-3321):
+// 2 hq = |u|^2 and p / rho = 1 / (2 beta).
+template <int DIM>
+__device__ __forceinline__ double node_speed(const Node<DIM> &n, double gamma) {
+  return root(2.0 * n.hq) + root(0.5 * gamma * rcp(n.beta));
+}
+
 // Conservative -> entropy variables.  s = ln((gamma-1) rho e) - gamma ln rho
 // (the reference evaluates ln((gamma-1) rho e / rho^gamma)).
 template <int DIM>
@@ -216,9 +331,9 @@ __device__ __forceinline__ void entropy_vars(const double (&U)[DIM + 2], double 
   const double rho = U[0], E = U[DIM + 1];
   double mm = U[1] * U[1];
   for (int d = 1; d < DIM; ++d) mm = mm + U[1 + d] * U[1 + d];
-  const double rhoe = E - 0.5 * mm / rho;
-  const double s = log((gamma - 1.0) * rhoe) - gamma * log(rho);
-  const double invrhoe = 1.0 / rhoe;
+  const double rhoe = E - quot(0.5 * mm, rho, rcp(rho));
+  const double s = ln((gamma - 1.0) * rhoe) - gamma * ln(rho);
+  const double invrhoe = rcp(rhoe);
   V[0] = (-E) * invrhoe + ((gamma + 1.0) - s);
   for (int d = 0; d < DIM; ++d) V[1 + d] = U[1 + d] * invrhoe;
   V[DIM + 1] = (-rho) * invrhoe;
@@ -233,9 +348,9 @@ __device__ __forceinline__ void conservative_vars(const double (&V)[DIM + 2], do
   const double vl = V[DIM + 1];
   double vv = V[1] * V[1];
   for (int d = 1; d < DIM; ++d) vv = vv + V[1 + d] * V[1 + d];
-  const double h = vv / (2.0 * vl);
+  const double h = quot(0.5 * vv, vl, rcp(vl));
   const double s = gamma - V[0] + h;
-  const double rhoe = exp((lgm1 - gamma * log(-vl) - s) / (gamma - 1.0));
+  const double rhoe = expo(quot(lgm1 - gamma * ln(-vl) - s, gamma - 1.0, rcp(gamma - 1.0)));
   U[0] = rhoe * (-vl);
   for (int d = 0; d < DIM; ++d) U[1 + d] = rhoe * V[1 + d];
   U[DIM + 1] = rhoe * (1.0 - h);
@@ -452,8 +567,8 @@ __device__ __forceinline__ double wavespeed(const double (&U)[DIM + 2], double g
     uu = uu + v[d] * v[d];
   }
   const double p = gm1 * (U[DIM + 1] - 0.5 * U[0] * uu);
-  const double su = sqrt(uu);
-  const double c = sqrt(gamma * p * irho);
+  const double su = root(uu);
+  const double c = root(gamma * p * irho);
   // d|u|: d(|u|)/du_d = u_d/|u| (0 at rest); u_d = m_d/rho
   const double isu = su > 0.0 ? rcp(su) : 0.0;
   // c^2 = gamma p / rho: d(c)/dq = (gamma/(2c)) d(p/rho)/dq
@@ -503,8 +618,8 @@ __device__ __forceinline__ void conservative_vars_vjp(const double (&V)[DIM + 2]
   const double ivl = rcp(vl);
   const double h = 0.5 * vv * ivl;
   const double s = gamma - V[0] + h;
-  const double igm1 = 1.0 / (gamma - 1.0);
-  const double rhoe = exp((lgm1 - gamma * log(-vl) - s) * igm1);
+  const double igm1 = rcp(gamma - 1.0);
+  const double rhoe = expo((lgm1 - gamma * ln(-vl) - s) * igm1);
   double rhoeb = Ub[0] * (-vl) + Ub[NF - 1] * (1.0 - h);
   for (int d = 0; d < DIM; ++d) rhoeb = rhoeb + Ub[1 + d] * V[1 + d];
   double vlb = -Ub[0] * rhoe;
