@@ -104,7 +104,14 @@ template <int DIM_, int NQ_, int NFQ_> struct Shape {
   // 64): the volume-face block is walked by face point, every lane busy.
   static constexpr bool COLVF = R == 1 && TPW == 1 && NFN == WAVE && NQ < WAVE;
   static constexpr int WS_C = COLVF ? 2 * NQ * NFN : 0;   // its weights
-  static constexpr int WS = WS_D + WS_W + WS_R + WS_C;
+  // the walk of wadges_wide.hpp: pairs, their weights where none of the tables
+  // above has them in its order (faces taken in parts), their codes (4 bytes)
+  static constexpr int WALK = COLVF || R > 1 || NQ <= NFN ? NQ * NFN : L * NQ;
+  static constexpr bool PARTS = R == 1 && NQ <= NFN && !COLVF &&
+                                (DIM == 2 ? (NQ + NFQ - 1) / NFQ == 2 : (NQ + NFQ - 1) / NFQ <= 2);
+  static constexpr int WS_V = PARTS ? 2 * WALK : 0;
+  static constexpr int WS_K = (WALK + 1) / 2;
+  static constexpr int WS = WS_D + WS_W + WS_R + WS_C + WS_V + WS_K;
   static_assert(R == 1 || (NQ <= NFN && LPE <= NFQ), "R > 1 needs one element's lanes on one face");
 };
 
@@ -158,6 +165,58 @@ template <class S> constexpr int face_parts() {
   return (face_chunked<S>() && S::NFACES == 4 && face_groups<S>() <= 2) ? 2 : 1;
 }
 
+// Order of the volume-face block of the fused stage as a list: steps s of P pairs
+// each; slot p of a step is the pair of row i and face point fn.  A row adds its
+// contributions in the order of the steps, a face point too (with two rows per
+// lane, the sum of a lane's two rows at a time).  Step s, slot p has its weights
+// +1/2 VqLq and -1/2 VfPq at W1 and W2 + s * P + p of the workspace and its code,
+// i + 256 fn + 65536 face, at 4-byte slot s * P + p from CODES on; NONE: no pair.
+template <class S> struct VfWalk {
+  static constexpr bool COL = S::COLVF;                  // slots are face points
+  static constexpr int P = COL ? S::NFN : S::NQ;
+  static constexpr int STEPS = COL ? S::NQ : (S::R > 1 ? S::NFN : vf_steps<S>());
+  static constexpr bool CHUNKED = !COL && S::R == 1 && face_chunked<S>();
+  static constexpr int FH = S::NFACES / face_parts<S>();  // faces per part
+  static constexpr int W1 = S::WS_D + (COL ? S::WS_W + S::WS_R
+                                           : (S::R > 1 ? S::WS_W : (S::PARTS ? S::WS_W + S::WS_R + S::WS_C : 0)));
+  static constexpr int W2 = W1 + STEPS * P;
+  static constexpr int CODES = S::WS - S::WS_K;
+  static constexpr uint32_t NONE = ~0u;
+  static_assert(S::WALK == STEPS * P, "walk tables");
+  static_assert(S::PARTS == (CHUNKED && face_parts<S>() > 1), "weights in the order of the parts");
+
+  static __device__ __forceinline__ bool pair(int s, int p, int &i, int &fn) {
+    if constexpr (COL) {
+      i = (p < S::NQ ? p : p - S::NQ) + s;
+      if (i >= S::NQ) i -= S::NQ;
+      fn = p;
+      return true;
+    } else if constexpr (S::R > 1) {
+      i = p;
+      const int face = s / S::NFQ;
+      int q = (i < S::LPE ? i : i - S::LPE) + (s - face * S::NFQ);
+      if (q >= S::NFQ) q -= S::NFQ;
+      fn = face * S::NFQ + q;
+      return true;
+    } else if constexpr (CHUNKED) {
+      i = p;
+      const int c = s / S::NFQ, m = s - c * S::NFQ;       // c = part * FH + u
+      const int h = c / FH;
+      const int g = i / S::NFQ, o = i - g * S::NFQ;
+      const int fh = (c - h * FH + g) % FH;
+      int node = o + m;
+      if (node >= S::NFQ) node -= S::NFQ;
+      fn = (h * FH + fh) * S::NFQ + node;
+      return true;
+    } else {
+      i = p;
+      fn = i + s;
+      if (fn >= S::L) fn -= S::L;
+      return fn < S::NFN;
+    }
+  }
+};
+
 // ------------------------------------------------------------------ operator prep
 
 template <class S>
@@ -184,7 +243,7 @@ __global__ void prep_vol_tables(const double *__restrict__ Drq, const double *__
     double v = 0.0;
     if (f < NFN) v = s == 0 ? 0.5 * VqLq[i + f * NQ] : -0.5 * VfPq[f + i * NFN];
     ws[idx] = v;
-  } else if (S::R > 1 && idx >= S::WS_D + S::WS_W && idx < S::WS) {
+  } else if (S::R > 1 && idx >= S::WS_D + S::WS_W && idx < S::WS_D + S::WS_W + S::WS_R) {
     // face walk of R > 1: step t = face * NFQ + m, row i on lane l = i mod LPE
     // visits point (l + m) mod NFQ of that face
     const int k = idx - S::WS_D - S::WS_W;
@@ -195,7 +254,8 @@ __global__ void prep_vol_tables(const double *__restrict__ Drq, const double *__
     if (q >= S::NFQ) q -= S::NFQ;
     const int f = (t / S::NFQ) * S::NFQ + q;
     ws[idx] = s == 0 ? 0.5 * VqLq[i + f * NQ] : -0.5 * VfPq[f + i * NFN];
-  } else if (S::COLVF && idx >= S::WS_D + S::WS_W + S::WS_R && idx < S::WS) {
+  } else if (S::COLVF && idx >= S::WS_D + S::WS_W + S::WS_R &&
+             idx < S::WS_D + S::WS_W + S::WS_R + S::WS_C) {
     // face-point walk: step t, lane L (face point L) visits row (L mod NQ + t) mod NQ
     const int k = idx - S::WS_D - S::WS_W - S::WS_R;
     const int L = k % NFN;
@@ -204,6 +264,19 @@ __global__ void prep_vol_tables(const double *__restrict__ Drq, const double *__
     int i = L % NQ + t;
     if (i >= NQ) i -= NQ;
     ws[idx] = s == 0 ? 0.5 * VqLq[i + L * NQ] : -0.5 * VfPq[L + i * NFN];
+  } else if (S::PARTS && idx >= VfWalk<S>::W1 && idx < VfWalk<S>::W1 + S::WS_V) {
+    const int k = idx - VfWalk<S>::W1;
+    const int s = k / S::WALK;
+    int i, f;
+    VfWalk<S>::pair((k % S::WALK) / NQ, k % NQ, i, f);
+    ws[idx] = s == 0 ? 0.5 * VqLq[i + f * NQ] : -0.5 * VfPq[f + i * NFN];
+  } else if (idx >= VfWalk<S>::CODES && idx < S::WS) {
+    uint32_t *code = (uint32_t *)(ws + VfWalk<S>::CODES);
+    for (int k = 2 * (idx - VfWalk<S>::CODES); k < 2 * (idx - VfWalk<S>::CODES) + 2 && k < S::WALK; ++k) {
+      int i, f;
+      const bool ok = VfWalk<S>::pair(k / VfWalk<S>::P, k % VfWalk<S>::P, i, f);
+      code[k] = ok ? (uint32_t)(i + 256 * f + 65536 * (f / S::NFQ)) : VfWalk<S>::NONE;
+    }
   }
 }
 
@@ -1389,6 +1462,8 @@ __attribute__((amdgpu_waves_per_eu(vol_waves_min<S>(), vol_waves<S>()))) stage_k
                 threadIdx.x, s_nref, smem);
 }
 
+#include "wadges_wide.hpp"
+
 #include "wadges_adjoint.hpp"
 
 // ------------------------------------------------------------------ dispatch
@@ -1462,6 +1537,7 @@ struct Ops {
                   const double *, const double *, double *, hipStream_t);
   int (*prep)(const double *, const double *, const double *, const double *, const double *,
               double *, hipStream_t);
+  void (*wide)(int, int (&)[2]);
   int ws_doubles;
   int stage_smem;  // dynamic LDS bytes of one fused-stage workgroup
   int stage_tpw;   // elements per fused-stage workgroup
@@ -1478,6 +1554,7 @@ struct wadges_plan {
   // device (wadges_diagnostics_noalloc).
   double *scratch_addr;
   wadges::Ops ops;
+  int wide_k[2];  // largest meshes of the wide launches of the fused stage
   // Operator pointers the tables of the calls outside capture (ws[0, WS)) were
   // prepared from (null: not prepared).
   mutable const double *tab_src[5];
@@ -1591,8 +1668,29 @@ template <class S> int stage_impl(const wadges_plan *p, int K, const double *vge
               tab,    VqLq,   VqPq,    VfPq,   Jq,     fa,      fb,   fdt,
               Qf_in,  Qf_out, rhsQ,    resQ,   Q,      rhsQ_in, resQ_in, Q_in,
               g,      g - 1.0, 1.0 / (2.0 * (g - 1.0)), 0.25 * p->tau, std::log(g - 1.0)};
-  stage_kernel<S><<<blocks, WAVE, smem, st>>>(A);
+  using Small = typename WideChoice<S>::Small;
+  using Large = typename WideChoice<S>::Large;
+  if (K <= p->wide_k[0])
+    stage_wide<Small><<<(K + Small::E - 1) / Small::E, Small::T, Small::bytes, st>>>(A);
+  else if (K <= p->wide_k[1])
+    stage_wide<Large><<<(K + Large::E - 1) / Large::E, Large::T, Large::bytes, st>>>(A);
+  else
+    stage_kernel<S><<<blocks, WAVE, smem, st>>>(A);
   return hip_check(hipGetLastError());
+}
+
+// Largest meshes of the two wide launches on a device of `cus` CUs (0: none).
+template <class S> void wide_limits(int cus, int (&k)[2]) {
+  using Small = typename WideChoice<S>::Small;
+  using Large = typename WideChoice<S>::Large;
+  int occ = 0;
+  k[0] = k[1] = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Small>, Small::T,
+                                                   Small::bytes) == hipSuccess)
+    k[0] = std::min(2, occ * Small::E) * cus;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Large>, Large::T,
+                                                   Large::bytes) == hipSuccess)
+    k[1] = occ * Large::E * cus;
 }
 
 template <class S> int diag_impl(const wadges_plan *p, int K, const double *wq, const double *Jq,
@@ -1717,7 +1815,7 @@ template <int DIM, int NQ, int NFQ> constexpr Instance make_instance(int N) {
                   Ops{&vol_impl<S>, &surf_impl<S>, &update_impl<S>, &stage_impl<S>,
                       &stage_vjp_impl<S>, &diag_impl<S>,
                       &rhs_vjp_impl<S>, &update_vjp_impl<S>, &proj_vjp_impl<S>, &prep_impl<S>,
-                      S::WS, stage_smem_bytes<S>(), S::TPW}};
+                      &wide_limits<S>, S::WS, stage_smem_bytes<S>(), S::TPW}};
 }
 
 // (dim, N, Nq, Nfq): quadrature of degree 2N, the point counts of the reference's
@@ -1795,6 +1893,10 @@ int wadges_plan_create(wadges_plan **plan, int dim, int N, int Nq, int Nfq, doub
     delete p;
     return WADGES_EHIP;
   }
+  p->wide_k[0] = p->wide_k[1] = 0;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess)
+    inst->ops.wide(cus, p->wide_k);
   // the fixed diagnostics array of this device (looked up once per device; a
   // failure here is reported by wadges_diagnostics_noalloc, which retries)
   p->scratch_addr = nullptr;
