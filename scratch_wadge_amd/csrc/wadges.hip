@@ -106,11 +106,11 @@ template <int DIM_, int NQ_, int NFQ_> struct Shape {
   static constexpr int WS_C = COLVF ? 2 * NQ * NFN : 0;   // its weights
   // the walk of wadges_wide.hpp: pairs, their weights where none of the tables
   // above has them in its order (faces taken in parts), their codes (4 bytes)
-  static constexpr int WALK = COLVF || R > 1 || NQ <= NFN ? NQ * NFN : L * NQ;
+  static constexpr int WALK = COLVF || NQ <= NFN ? NQ * NFN : L * NQ;
   static constexpr bool PARTS = R == 1 && NQ <= NFN && !COLVF &&
                                 (DIM == 2 ? (NQ + NFQ - 1) / NFQ == 2 : (NQ + NFQ - 1) / NFQ <= 2);
   static constexpr int WS_V = PARTS ? 2 * WALK : 0;
-  static constexpr int WS_K = (WALK + 1) / 2;
+  static constexpr int WS_K = R > 1 ? 0 : (WALK + 1) / 2;
   static constexpr int WS = WS_D + WS_W + WS_R + WS_C + WS_V + WS_K;
   static_assert(R == 1 || (NQ <= NFN && LPE <= NFQ), "R > 1 needs one element's lanes on one face");
 };
@@ -166,19 +166,18 @@ template <class S> constexpr int face_parts() {
 }
 
 // Order of the volume-face block of the fused stage as a list: steps s of P pairs
-// each; slot p of a step is the pair of row i and face point fn.  A row adds its
-// contributions in the order of the steps, a face point too (with two rows per
-// lane, the sum of a lane's two rows at a time).  Step s, slot p has its weights
-// +1/2 VqLq and -1/2 VfPq at W1 and W2 + s * P + p of the workspace and its code,
+// each; slot p of a step is the pair of row i and face point fn (one row per lane).  A row adds its
+// contributions in the order of the steps, a face point too.  Step s, slot p has its
+// weights +1/2 VqLq and -1/2 VfPq at W1 and W2 + s * P + p of the workspace and its code,
 // i + 256 fn + 65536 face, at 4-byte slot s * P + p from CODES on; NONE: no pair.
 template <class S> struct VfWalk {
   static constexpr bool COL = S::COLVF;                  // slots are face points
   static constexpr int P = COL ? S::NFN : S::NQ;
-  static constexpr int STEPS = COL ? S::NQ : (S::R > 1 ? S::NFN : vf_steps<S>());
-  static constexpr bool CHUNKED = !COL && S::R == 1 && face_chunked<S>();
+  static constexpr int STEPS = COL ? S::NQ : vf_steps<S>();
+  static constexpr bool CHUNKED = !COL && face_chunked<S>();
   static constexpr int FH = S::NFACES / face_parts<S>();  // faces per part
   static constexpr int W1 = S::WS_D + (COL ? S::WS_W + S::WS_R
-                                           : (S::R > 1 ? S::WS_W : (S::PARTS ? S::WS_W + S::WS_R + S::WS_C : 0)));
+                                           : (S::PARTS ? S::WS_W + S::WS_R + S::WS_C : 0));
   static constexpr int W2 = W1 + STEPS * P;
   static constexpr int CODES = S::WS - S::WS_K;
   static constexpr uint32_t NONE = ~0u;
@@ -190,13 +189,6 @@ template <class S> struct VfWalk {
       i = (p < S::NQ ? p : p - S::NQ) + s;
       if (i >= S::NQ) i -= S::NQ;
       fn = p;
-      return true;
-    } else if constexpr (S::R > 1) {
-      i = p;
-      const int face = s / S::NFQ;
-      int q = (i < S::LPE ? i : i - S::LPE) + (s - face * S::NFQ);
-      if (q >= S::NFQ) q -= S::NFQ;
-      fn = face * S::NFQ + q;
       return true;
     } else if constexpr (CHUNKED) {
       i = p;
@@ -264,18 +256,21 @@ __global__ void prep_vol_tables(const double *__restrict__ Drq, const double *__
     int i = L % NQ + t;
     if (i >= NQ) i -= NQ;
     ws[idx] = s == 0 ? 0.5 * VqLq[i + L * NQ] : -0.5 * VfPq[L + i * NFN];
-  } else if (S::PARTS && idx >= VfWalk<S>::W1 && idx < VfWalk<S>::W1 + S::WS_V) {
-    const int k = idx - VfWalk<S>::W1;
-    const int s = k / S::WALK;
-    int i, f;
-    VfWalk<S>::pair((k % S::WALK) / NQ, k % NQ, i, f);
-    ws[idx] = s == 0 ? 0.5 * VqLq[i + f * NQ] : -0.5 * VfPq[f + i * NFN];
-  } else if (idx >= VfWalk<S>::CODES && idx < S::WS) {
-    uint32_t *code = (uint32_t *)(ws + VfWalk<S>::CODES);
-    for (int k = 2 * (idx - VfWalk<S>::CODES); k < 2 * (idx - VfWalk<S>::CODES) + 2 && k < S::WALK; ++k) {
+  } else if constexpr (S::R == 1) {
+    using Vf = VfWalk<S>;
+    if (S::PARTS && idx >= Vf::W1 && idx < Vf::W1 + S::WS_V) {
+      const int k = idx - Vf::W1;
+      const int s = k / S::WALK;
       int i, f;
-      const bool ok = VfWalk<S>::pair(k / VfWalk<S>::P, k % VfWalk<S>::P, i, f);
-      code[k] = ok ? (uint32_t)(i + 256 * f + 65536 * (f / S::NFQ)) : VfWalk<S>::NONE;
+      Vf::pair((k % S::WALK) / NQ, k % NQ, i, f);
+      ws[idx] = s == 0 ? 0.5 * VqLq[i + f * NQ] : -0.5 * VfPq[f + i * NFN];
+    } else if (idx >= Vf::CODES && idx < S::WS) {
+      uint32_t *code = (uint32_t *)(ws + Vf::CODES);
+      for (int k = 2 * (idx - Vf::CODES); k < 2 * (idx - Vf::CODES) + 2 && k < S::WALK; ++k) {
+        int i, f;
+        const bool ok = Vf::pair(k / Vf::P, k % Vf::P, i, f);
+        code[k] = ok ? (uint32_t)(i + 256 * f + 65536 * (f / S::NFQ)) : Vf::NONE;
+      }
     }
   }
 }
@@ -344,10 +339,17 @@ struct WaveCtx {
   double *smem;        // the workgroup's dynamic LDS (team t at t * per_elem)
 };
 
+// With two rows per lane (3D N = 3) the sums are kept in the parts that the waves of
+// wadges_team.hpp form: the steps of the volume-volume block in NFACES equal groups
+// (in a group the lanes' first rows take their steps, then add their own sums, then
+// the second rows), then one part per face.  A row's total is ((((T0 + T1) + T2) +
+// T3) + P0) + ... + P3.
+
 // The volume term of one element (both coupling blocks).  Lane l of the
 // element's team owns rows l + r * LPE (r < R, those below NQ).  On return
 // acc[r] holds the register part of its row r, accV the LDS part (partner
-// contributions), accF the face rows (rhsQf).  Uq is the element's projected
+// contributions; with R > 1 the whole sum, and acc is zero), accF the face rows
+// (rhsQf).  Uq is the element's projected
 // volume state, vg its volume geofacs; the face state and geofacs of the wave's
 // elements come through wc.  Every lane of the workgroup must call this
 // (barriers).
@@ -421,24 +423,24 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
   int vv_steps = TVT;
   if constexpr (ROLLED) vv_steps = opaque_bound(TVT);
   if (valid) {
-    // With R > 1 the operator entries of step t + 1 are loaded while step t
-    // computes (one row per lane has no registers to spare for it).  (Two
-    // buffers used in turn, as in the face walk below, spilled here.)
-    constexpr bool PIPE = R > 1 || DIM == 2;
+    // In 2D the operator entries of step t + 1 are loaded while step t computes
+    // (the 3D shapes have no registers to spare for it).
+    constexpr bool PIPE = DIM == 2;
     const double *Dfw = ws;
     const double *Dbw = ws + DIM * TVT * NQ;
     int iw[R];                        // table row (row 0's for rows that do not exist)
     for (int r = 0; r < R; ++r) iw[r] = rv[r] ? l + r * LPE : 0;
-    auto fetch = [&](int t, double (&Df)[R][DIM], double (&Db)[R][DIM]) {
+    // one: that row only (every row if negative)
+    auto fetch = [&](int t, double (&Df)[R][DIM], double (&Db)[R][DIM], int one = -1) {
       for (int r = 0; r < R; ++r)
-        for (int q = 0; q < DIM; ++q) {
+        for (int q = 0; q < DIM && (one < 0 || r == one); ++q) {
           Df[r][q] = ld_off(Dfw, (unsigned)((q * TVT + t) * NQ + iw[r]));
           Db[r][q] = ld_off(Dbw, (unsigned)((q * TVT + t) * NQ + iw[r]));
         }
     };
-    auto vv_step = [&](int t, const double (&Df)[R][DIM], const double (&Db)[R][DIM]) {
+    auto vv_step = [&](int t, const double (&Df)[R][DIM], const double (&Db)[R][DIM], int one = -1) {
       for (int r = 0; r < R; ++r) {
-        if (!rv[r]) continue;
+        if (!rv[r] || (one >= 0 && r != one)) continue;
         const int i = l + r * LPE;
         if (2 * t == NQ && i >= NQ / 2) continue;  // even NQ: middle pair once
         int j = i + t;
@@ -464,7 +466,41 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
       }
     };
     {
-      if constexpr (PIPE) {
+      if constexpr (R > 1) {
+        constexpr int TG = TVT / S::NFACES;
+        static_assert(TVT % S::NFACES == 0 && NQ % 2 == 1 && TG > 1, "equal groups, every row a partner");
+        double tot[R][NFLD];
+        for (int r = 0; r < R; ++r)
+          for (int f = 0; f < NFLD; ++f) tot[r][f] = 0.0;
+#pragma unroll 1
+        for (int g = 0; g < S::NFACES; ++g) {
+          for (int r = 0; r < R; ++r) {
+#pragma unroll 1
+            for (int t = g * TG; t < (g + 1) * TG; ++t) {
+              double Df[R][DIM], Db[R][DIM];
+              fetch(t, Df, Db, r);
+              vv_step(t, Df, Db, r);
+            }
+            if (!rv[r]) continue;
+            for (int f = 0; f < NFLD; ++f) {
+              lds_add(&accV[f * NQ + l + r * LPE], acc[r][f]);
+              acc[r][f] = 0.0;
+            }
+          }
+          // the group's sum joins the total; its accumulator starts anew
+          for (int r = 0; r < R; ++r) {
+            if (!rv[r]) continue;
+            for (int f = 0; f < NFLD; ++f) {
+              double *a = &accV[f * NQ + l + r * LPE];
+              tot[r][f] += *a;
+              *a = 0.0;
+            }
+          }
+        }
+        for (int r = 0; r < R; ++r)
+          if (rv[r])
+            for (int f = 0; f < NFLD; ++f) accV[f * NQ + l + r * LPE] = tot[r][f];
+      } else if constexpr (PIPE) {
         double nDf[R][DIM], nDb[R][DIM];
         fetch(0, nDf, nDb);
         for (int t = 0; t < vv_steps; ++t) {
@@ -700,6 +736,13 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
           vf_step(m, s0);
           if (m + 2 < NFQ) fetch(m + 2, s0);
           vf_step(m + 1, s1);
+        }
+        for (int r = 0; r < R; ++r) {
+          if (!rv[r]) continue;
+          for (int f = 0; f < NFLD; ++f) {
+            accV[f * NQ + l + r * LPE] += acc[r][f];
+            acc[r][f] = 0.0;
+          }
         }
       } else {
         const int i = l;
@@ -1462,6 +1505,7 @@ __attribute__((amdgpu_waves_per_eu(vol_waves_min<S>(), vol_waves<S>()))) stage_k
                 threadIdx.x, s_nref, smem);
 }
 
+#include "wadges_team.hpp"
 #include "wadges_wide.hpp"
 
 #include "wadges_adjoint.hpp"
@@ -1616,9 +1660,15 @@ template <class S> int vol_impl(const wadges_plan *p, int K, const double *vgeo,
   static_assert(TPW >= 1, "Nq must fit in one wave");
   const size_t smem = (size_t)TPW * VolSmem<S>::per_elem * sizeof(double);
   const int blocks = (K + TPW - 1) / TPW;
-  vol_kernel<S><<<blocks, WAVE, smem, st>>>(K, vgeo, vfgeo, nrJ, nsJ, ntJ, tab, Qf, rhsQ,
-                                                 rhsQf, p->gamma - 1.0,
-                                                 1.0 / (2.0 * (p->gamma - 1.0)));
+  const double gm1 = p->gamma - 1.0;
+  if constexpr (S::R > 1) {
+    using X = Team<S>;
+    team_vol_kernel<S><<<(K + X::E - 1) / X::E, X::T, X::bytes, st>>>(K, vgeo, vfgeo, nrJ, nsJ, ntJ, tab, Qf,
+                                                              rhsQ, rhsQf, gm1, 1.0 / (2.0 * gm1));
+  } else {
+    vol_kernel<S><<<blocks, WAVE, smem, st>>>(K, vgeo, vfgeo, nrJ, nsJ, ntJ, tab, Qf, rhsQ, rhsQf,
+                                              gm1, 1.0 / (2.0 * gm1));
+  }
   return hip_check(hipGetLastError());
 }
 
@@ -1668,29 +1718,36 @@ template <class S> int stage_impl(const wadges_plan *p, int K, const double *vge
               tab,    VqLq,   VqPq,    VfPq,   Jq,     fa,      fb,   fdt,
               Qf_in,  Qf_out, rhsQ,    resQ,   Q,      rhsQ_in, resQ_in, Q_in,
               g,      g - 1.0, 1.0 / (2.0 * (g - 1.0)), 0.25 * p->tau, std::log(g - 1.0)};
-  using Small = typename WideChoice<S>::Small;
-  using Large = typename WideChoice<S>::Large;
-  if (K <= p->wide_k[0])
-    stage_wide<Small><<<(K + Small::E - 1) / Small::E, Small::T, Small::bytes, st>>>(A);
-  else if (K <= p->wide_k[1])
-    stage_wide<Large><<<(K + Large::E - 1) / Large::E, Large::T, Large::bytes, st>>>(A);
-  else
-    stage_kernel<S><<<blocks, WAVE, smem, st>>>(A);
+  if constexpr (S::R > 1) {
+    using X = Team<S>;
+    team_stage_kernel<S><<<(K + X::E - 1) / X::E, X::T, X::bytes, st>>>(A);
+  } else {
+    using Small = typename WideChoice<S>::Small;
+    using Large = typename WideChoice<S>::Large;
+    if (K <= p->wide_k[0])
+      stage_wide<Small><<<(K + Small::E - 1) / Small::E, Small::T, Small::bytes, st>>>(A);
+    else if (K <= p->wide_k[1])
+      stage_wide<Large><<<(K + Large::E - 1) / Large::E, Large::T, Large::bytes, st>>>(A);
+    else
+      stage_kernel<S><<<blocks, WAVE, smem, st>>>(A);
+  }
   return hip_check(hipGetLastError());
 }
 
 // Largest meshes of the two wide launches on a device of `cus` CUs (0: none).
 template <class S> void wide_limits(int cus, int (&k)[2]) {
-  using Small = typename WideChoice<S>::Small;
-  using Large = typename WideChoice<S>::Large;
-  int occ = 0;
   k[0] = k[1] = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Small>, Small::T,
-                                                   Small::bytes) == hipSuccess)
-    k[0] = std::min(2, occ * Small::E) * cus;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Large>, Large::T,
-                                                   Large::bytes) == hipSuccess)
-    k[1] = occ * Large::E * cus;
+  if constexpr (S::R == 1) {
+    using Small = typename WideChoice<S>::Small;
+    using Large = typename WideChoice<S>::Large;
+    int occ = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Small>, Small::T,
+                                                     Small::bytes) == hipSuccess)
+      k[0] = std::min(2, occ * Small::E) * cus;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Large>, Large::T,
+                                                     Large::bytes) == hipSuccess)
+      k[1] = occ * Large::E * cus;
+  }
 }
 
 template <class S> int diag_impl(const wadges_plan *p, int K, const double *wq, const double *Jq,

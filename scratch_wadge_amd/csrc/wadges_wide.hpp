@@ -4,8 +4,8 @@
 //
 // stage_body packs several elements into a wave and gives each lane a row, which
 // then walks its partners one after the other: few instructions per element,
-// but a wave takes its whole walk (3D N = 3: 120 pair fluxes in a row) however
-// few waves there are.  Here a workgroup of W waves holds E elements and every
+// but a wave takes its whole walk (3D N = 4: 67 pair fluxes in a row) however few
+// waves there are.  Here a workgroup of W waves holds E elements and every
 // lane evaluates one pair at a time, so the walk is E * pairs / (64 W) long.  The
 // contributions go to LDS and are then added, one lane per (row, field) and per
 // (face point, field), in the order in which stage_body adds them: the results
@@ -19,6 +19,7 @@ template <class S_, int E_, int W_, int CV_, int CF_> struct Wide {
   using S = S_;
   static constexpr int E = E_, W = W_, CV = CV_, CF = CF_;
   static constexpr int T = WAVE * W;
+  static_assert(S::R == 1, "one row per lane in the packed stage");
   using Vf = VfWalk<S>;
   static constexpr int CVP = CV * S::NQ, CFP = CF * Vf::P;
   // per-element LDS (doubles): volume records, normal parts of the rows on each
@@ -50,7 +51,6 @@ template <class S_, int E_, int W_, int CV_, int CF_> struct Wide {
 //   2D N = 5   K = 512    26.5 / 16.9   1,058  27.1 / 30.3
 //   3D N = 1   K = 384    21.5 / 9.8    6,000  24.6 / 16.8   10,368  26.8 / 26.4
 //   3D N = 2   K = 162    25.3 / 11.2     750  25.6 / 13.4    1,296  26.2 / 24.0
-//   3D N = 3   K = 162    54.4 / 18.4     750  54.6 / 28.0    1,296  56.3 / 51.0
 //   3D N = 4   K = 384    47.3 / 36.0     750  49.1 / 45.1    1,296  67.8 / 83.9
 template <class S> struct WideChoice;
 template <> struct WideChoice<Shape<2, 3, 2>> {
@@ -80,10 +80,6 @@ template <> struct WideChoice<Shape<3, 4, 3>> {
 template <> struct WideChoice<Shape<3, 11, 6>> {
   using Small = Wide<Shape<3, 11, 6>, 1, 2, 6, 24>;
   using Large = Small;
-};
-template <> struct WideChoice<Shape<3, 23, 12>> {
-  using Small = Wide<Shape<3, 23, 12>, 1, 4, 12, 12>;
-  using Large = Wide<Shape<3, 23, 12>, 1, 2, 12, 24>;
 };
 template <> struct WideChoice<Shape<3, 44, 16>> {
   using Small = Wide<Shape<3, 44, 16>, 1, 4, 6, 4>;
@@ -413,7 +409,7 @@ stage_wide(StageArgs args) {
 #pragma unroll
         for (int sl = 0; sl < CF; ++sl) {
           const int at = sl * Vf::P + si[x];
-          if constexpr (Vf::CHUNKED || S::R > 1) {
+          if constexpr (Vf::CHUNKED) {
             acc[x] += w1[at] * F[at];
           } else {
             int fn = si[x] + s0 + sl;         // no pair beyond the face points
@@ -434,22 +430,6 @@ stage_wide(StageArgs args) {
         for (int sl = 0; sl < CF; ++sl) {
           const int at = sl * Vf::P + gn[x];
           accf[x] += w2[at] * F[at];
-        }
-      } else if constexpr (S::R > 1) {
-        static_assert(CF % NFQ == 0, "whole faces at a time");
-        const int hl = face - s0 / NFQ;       // this face among those of the chunk
-        if (hl < 0 || hl >= CF / NFQ) continue;
-        int l = q;                            // the lane of stage_body that visits the point
-#pragma unroll
-        for (int m = 0; m < NFQ; ++m) {
-          const int at = (hl * NFQ + m) * Vf::P + l;
-          const bool second = l + S::LPE < NQ;
-          const int at2 = second ? at + S::LPE : at;
-          double sF = 0.0;
-          sF += w2[at] * F[at];
-          const double sF2 = sF + w2[at2] * F[at2];
-          accf[x] += second ? sF2 : sF;
-          l = l == 0 ? NFQ - 1 : l - 1;
         }
       } else if constexpr (Vf::CHUNKED) {
         constexpr int GR = face_groups<S>(), FH = Vf::FH;

@@ -1,7 +1,8 @@
-"""The fused stage of small meshes (an element's pairs spread over a workgroup)
-against the packed one, which ensembles run whatever their size: equal bit for
-bit for every shape, on meshes of both launch shapes, with full and partly filled
-last workgroups, on the initial state and on a state with both log-mean branches."""
+"""The fused stage of small meshes (an element's pairs spread over a workgroup), and
+of 3D N = 3 on every mesh (a wave per face), against the packed one, which
+ensembles run whatever their size: equal bit for bit for every shape, on meshes of
+both launch shapes, with full and partly filled last workgroups, on the initial
+state and on a state with both log-mean branches."""
 
 import numpy as np
 import pytest
