@@ -118,7 +118,7 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
   if (valid) {
     double U[NFLD];
     for (int f = 0; f < NFLD; ++f) U[f] = Uq[kk * NQ * NFLD + f * NQ + i];
-    me = make_node<DIM>(U, gm1);
+    me = make_node<DIM, false>(U, gm1);
     for (int c = 0; c < NG; ++c) hG[c] = 0.5 * vgeo[kk * NQ * NG + c * NQ + i];
     store_node<DIM>(vrec, NQ, i, me);
     for (int c = 0; c < NG; ++c) vrec[(VS + c) * NQ + i] = hG[c];
@@ -129,10 +129,34 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
     for (int c = 0; c < NPB; ++c) gV[c * NQ + i] = 0.0;
   }
   __syncthreads();
+  // logarithms of the records only where the wave is not smooth (as in the forward
+  // volume term: a smooth wave's pairs all take the series branch)
+  const double rho_ref = smem[NPB * NQ], beta_ref = smem[NPB * NQ + (DIM + 1) * NQ];
+  const bool smooth_v = uniform_flag(
+      wave_all(!valid || in_smooth_band<DIM>(me.rho, me.beta, rho_ref, beta_ref)));
+  auto own_logs = [&]() {
+    if (!valid) return;
+    me.lrho = ln(me.rho);
+    me.lbeta = ln(me.beta);
+  };
+  if (!smooth_v) {
+    own_logs();
+    if (valid) {
+      vrec[(DIM + 2) * NQ + i] = me.lrho;
+      vrec[(DIM + 3) * NQ + i] = me.lbeta;
+    }
+    __syncthreads();
+  }
+  // Loops kept rolled where unrolled completely they spill or leave one wave per SIMD
+  // (3D N = 1, 2; 2D from N = 3 on): 3D N = 2, K = 16,464, 101 -> 81 us; 2D N = 4, K =
+  // 8,192, 36 -> 30 us.  The other shapes lose 5 % by it.
+  constexpr bool ROLLED = DIM == 3 ? NQ <= 11 : NQ >= 12;
+  auto bound = [](int v) { return ROLLED ? opaque_bound(v) : v; };
   if (valid) {
     const double *Dfw = ws;
     const double *Dbw = ws + DIM * TVT * NQ;
-    for (int t = 0; t < TVT; ++t) {
+    const int steps = bound(TVT);
+    for (int t = 0; t < steps; ++t) {
       if (2 * t > NQ) break;
       if (2 * t == NQ && i >= NQ / 2) continue;
       int j = i + t;
@@ -181,6 +205,7 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
   // ---------------- phase 2: face records, s_bar, volume-face pairs.  Face
   // point work of all teams is spread over the whole wave.
   auto team_base = [&](int t) { return smem + t * PER; };
+  bool ok_f = true;
   constexpr int OFF_FREC = NPB * NQ, OFF_SBF = OFF_FREC + FREC * NFN, OFF_GF = OFF_SBF + NFLD * NFN;
   for (int p = lane; p < TPW * NFN; p += WAVE) {
     const int t = p / NFN;
@@ -192,7 +217,9 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
     double *gft = team_base(t) + OFF_GF;
     double U[NFLD];
     for (int f = 0; f < NFLD; ++f) U[f] = Uf[kt * NFN * NFLD + f * NFN + fn];
-    store_node<DIM>(frt, NFN, fn, make_node<DIM>(U, gm1));
+    const Node<DIM> nf = make_node<DIM, false>(U, gm1);
+    ok_f = ok_f && in_smooth_band<DIM>(nf.rho, nf.beta, rho_ref, beta_ref);
+    store_node<DIM>(frt, NFN, fn, nf);
     const int face = fn / NFQ;
     for (int d = 0; d < DIM; ++d) {
       double b = 0.0;
@@ -204,6 +231,18 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
     for (int c = 0; c < NPB; ++c) gft[c * NFN + fn] = 0.0;
   }
   __syncthreads();
+  if (!uniform_flag(smooth_v && wave_all(ok_f))) {
+    if (smooth_v) own_logs();
+    for (int p = lane; p < TPW * NFN; p += WAVE) {
+      const int t = p / NFN;
+      const int fn = p - t * NFN;
+      if ((size_t)blockIdx.x * TPW + t >= (size_t)K) continue;
+      double *frt = team_base(t) + OFF_FREC;
+      frt[(DIM + 2) * NFN + fn] = ln(frt[fn]);
+      frt[(DIM + 3) * NFN + fn] = ln(frt[(DIM + 1) * NFN + fn]);
+    }
+    __syncthreads();
+  }
   if (valid) {
     const double *W1 = ws + S::WS_D;
     const double *W2 = W1 + T * NQ;
@@ -229,19 +268,21 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
     };
     if constexpr (face_chunked<S>()) {
       const int g = i / NFQ, o = i - (i / NFQ) * NFQ;
-      for (int c = 0; c < S::NFACES; ++c) {
+      const int faces = bound(S::NFACES), points = bound(NFQ);
+      for (int c = 0; c < faces; ++c) {
         int face = c + g;
         if (face >= S::NFACES) face -= S::NFACES;
         double a[DIM];
         own_normal(face, a);
-        for (int m = 0; m < NFQ; ++m) {
+        for (int m = 0; m < points; ++m) {
           int node = o + m;
           if (node >= NFQ) node -= NFQ;
           vf_pair(c * NFQ + m, face * NFQ + node, a);
         }
       }
     } else {
-      for (int t = 0; t < T; ++t) {
+      const int steps = bound(T);
+      for (int t = 0; t < steps; ++t) {
         const int fn = vf_partner<S>(t, i);
         if (fn >= NFN) continue;
         double a[DIM];
@@ -272,15 +313,15 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
       sbM[f] = sbt[f * NFN + fn];
       cons[f] = 0.0;
     }
-    const Node<DIM> a = make_node<DIM>(UM, gm1);
-    const Node<DIM> b = make_node<DIM>(UP, gm1);
+    const Node<DIM> a = make_node<DIM, false>(UM, gm1);
+    const Node<DIM> b = make_node<DIM, false>(UP, gm1);
     double hnM[DIM];
     for (int d = 0; d < DIM; ++d) hnM[d] = 0.5 * g[fn + d * NFN];
     const double sJM = g[fn + DIM * NFN];
     PrimBar<DIM> ga, gb;
     primbar_zero<DIM>(ga);
     primbar_zero<DIM>(gb);
-    flux_dot_vjp<DIM>(a, b, hnM, sbM, inv2gm1, ga, gb);
+    flux_dot_vjp<DIM, true>(a, b, hnM, sbM, inv2gm1, ga, gb);
     double dlM[NFLD], dlP[NFLD];
     const double lamM = wavespeed<DIM>(UM, gamma, gm1, dlM);
     const double lamP = wavespeed<DIM>(UP, gamma, gm1, dlP);
@@ -307,7 +348,7 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
       for (int f = 0; f < NFLD; ++f) sbP[f] = sbar[idP + (size_t)f * NFN];
       PrimBar<DIM> gx;
       primbar_zero<DIM>(gx);
-      flux_dot_vjp<DIM>(b, a, hnP, sbP, inv2gm1, gx, ga);
+      flux_dot_vjp<DIM, true>(b, a, hnP, sbP, inv2gm1, gx, ga);
       const double LfP = ltau * fmax(lamP, lamM) * sJP;
       double S2 = 0.0;
       for (int f = 0; f < NFLD; ++f) S2 = S2 + sbP[f] * (UM[f] - UP[f]);
@@ -548,7 +589,6 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
                 double lgm1) {
   constexpr int DIM = S::DIM, NQ = S::NQ, NFN = S::NFN, NFLD = S::NFLD;
   constexpr int EPB = 4 * TPW;
-  constexpr int MAXF = (NFN + NQ - 1) / NQ;
   __shared__ double bufA[EPB][NFLD][NQ];
   __shared__ double bufB[EPB][NFLD][NQ];
   __shared__ double bufF[EPB][NFLD][NFN];
@@ -561,7 +601,6 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
   const int k = blockIdx.x * EPB + e;
   const bool valid = active && k < K;
   const size_t base = (valid ? (size_t)k : 0) * NQ * NFLD;
-  const size_t basef = (valid ? (size_t)k : 0) * NFN * NFLD;
   double U[NFLD];
   if (valid) {
     double V[NFLD];
@@ -570,45 +609,47 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
     for (int f = 0; f < NFLD; ++f) bufA[e][f][i] = V[f];
   }
   __syncthreads();
-  double gq[NFLD], gfl[MAXF][NFLD];
+  // cotangents through u(VqPq v) and u(VfPq v), straight to LDS; the face points of the
+  // wave's elements spread over all its lanes
   if (valid) {
-    double V[NFLD], Ub[NFLD];
+    double V[NFLD], Ub[NFLD], g[NFLD];
     for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
+#pragma unroll 4
     for (int j = 0; j < NQ; ++j) {
       const double P = ld_off(VqPq, (unsigned)(i + j * NQ));
       for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[e][f][j];
     }
     for (int f = 0; f < NFLD; ++f) Ub[f] = uqb[base + i + f * NQ];
-    conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, gq);
-    for (int m = 0; m < MAXF; ++m) {
-      const int fn = i + m * NQ;
-      if (fn >= NFN) continue;
-      for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
-      for (int j = 0; j < NQ; ++j) {
-        const double P = ld_off(VfPq, (unsigned)(fn + j * NFN));
-        for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[e][f][j];
-      }
-      for (int f = 0; f < NFLD; ++f) Ub[f] = ufb[basef + fn + f * NFN];
-      conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, gfl[m]);
-    }
+    conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, g);
+    for (int f = 0; f < NFLD; ++f) bufB[e][f][i] = g[f];
   }
-  __syncthreads();
-  if (valid) {
-    for (int f = 0; f < NFLD; ++f) bufB[e][f][i] = gq[f];
-    for (int m = 0; m < MAXF; ++m) {
-      const int fn = i + m * NQ;
-      if (fn >= NFN) continue;
-      for (int f = 0; f < NFLD; ++f) bufF[e][f][fn] = gfl[m][f];
+  for (int p = wl; p < TPW * NFN; p += WAVE) {
+    const int t = p / NFN;
+    const int fn = p - t * NFN;
+    const int et = wave * TPW + t;
+    const int kt = blockIdx.x * EPB + et;
+    if (kt >= K) continue;
+    double V[NFLD], Ub[NFLD], g[NFLD];
+    for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < NQ; ++j) {
+      const double P = ld_off(VfPq, (unsigned)(fn + j * NFN));
+      for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[et][f][j];
     }
+    for (int f = 0; f < NFLD; ++f) Ub[f] = ufb[(size_t)kt * NFN * NFLD + fn + f * NFN];
+    conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, g);
+    for (int f = 0; f < NFLD; ++f) bufF[et][f][fn] = g[f];
   }
   __syncthreads();
   if (valid) {
     double vb[NFLD], Ub[NFLD];
     for (int f = 0; f < NFLD; ++f) vb[f] = 0.0;
+#pragma unroll 4
     for (int j = 0; j < NQ; ++j) {
       const double P = ld_off(VqPq, (unsigned)(j + i * NQ));
       for (int f = 0; f < NFLD; ++f) vb[f] += P * bufB[e][f][j];
     }
+#pragma unroll 4
     for (int fn = 0; fn < NFN; ++fn) {
       const double P = ld_off(VfPq, (unsigned)(fn + i * NFN));
       for (int f = 0; f < NFLD; ++f) vb[f] += P * bufF[e][f][fn];

@@ -438,53 +438,51 @@ __device__ __forceinline__ void logmean_partials(double a, double b, double la, 
 // tr = sum_k sum_d n_k[d] c_k[1+d], and the velocity derivative needs, per
 // direction, t_d = sum_k n_k[d] (c_k[0] + cm_k) + c_k[1+d] Un_k:
 // O(NT (DIM + NFLD)) work instead of the O(DIM^2 NFLD) of a dense Gb.
-template <int DIM, int NT>
+//
+// When every active lane of the wave takes the series branch of both log means
+// (smooth states), 1/F comes from the series of 1/F and every reciprocal of the pair
+// from one.  LAZY_LOGS: the nodes come without logarithms, which are then taken only
+// behind that test (the surface flux, whose nodes serve one pair per side).
+template <int DIM, int NT, bool LAZY_LOGS = false>
 __device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DIM> &b,
                                                const double (&n)[NT][DIM],
                                                const double (&c)[NT][DIM + 2], double inv2gm1,
                                                PrimBar<DIM> &ga, PrimBar<DIM> &gb) {
   constexpr int NF = DIM + 2;
-  double rl, rla, rlb, bl, bla, blb, isb, ibl;
-  const double sr = a.rho + b.rho, sb = a.beta + b.beta;
   constexpr double TH = (DIM == 3) ? 1.0e-4 : 1.0e-3;
+  const double sr = a.rho + b.rho, sb = a.beta + b.beta;
   const double dr = a.rho - b.rho, db = a.beta - b.beta;
-  bool series = false;
-  if constexpr (DIM == 3) {
-    // f of both log means from one reciprocal; when every active lane takes
-    // the series branch of both (smooth states), 1/F comes from the series of
-    // 1/F and every other reciprocal of the pair from that one.
-    const double q = rcp(sr * sb);
-    const double isr = sb * q;
-    const double isb1 = sr * q;
-    const double fr = dr * isr, fb = db * isb1;
-    const double ur = fr * fr, ub = fb * fb;
-    series = wave_all(ur < TH && ub < TH);
-    if (series) {
-      // l = s/(2F(u)); dl/da = 1/(2F) - l' b, dl/db = 1/(2F) + l' a with
-      // l' = 2 f F'(u) / (s F^2)  (the partials of the series branch)
-      auto partials = [&](double sa, double is, double f, double u, double x, double y,
-                          double &l, double &dx, double &dy, double &i2F) {
-        const double h = logmean_inv_series2<DIM>(u);          // 1/(2F)
-        const double Fp = 1.0 / 3.0 + u * (2.0 / 5.0 + u * (3.0 / 7.0));
-        l = sa * h;
-        const double t = 8.0 * f * Fp * is * h * h;           // 2 f F' / (s F^2)
-        dx = h - t * y;
-        dy = h + t * x;
-        i2F = h;
-      };
-      double hR, hB;
-      partials(sr, isr, fr, ur, a.rho, b.rho, rl, rla, rlb, hR);
-      partials(sb, isb1, fb, ub, a.beta, b.beta, bl, bla, blb, hB);
-      isb = isb1;
-      ibl = isb1 * logmean_series2<DIM>(ub);                  // 1/bl = 2F(u_beta)/sb
-      (void)hR;
-      (void)hB;
-    }
-  }
-  if (!series) {
-    logmean_partials<DIM>(a.rho, b.rho, a.lrho, b.lrho, rl, rla, rlb);
-    logmean_partials<DIM>(a.beta, b.beta, a.lbeta, b.lbeta, bl, bla, blb);
-    isb = rcp(sb);
+  // f of both log means from one reciprocal
+  const double q = rcp(sr * sb);
+  const double isr = sb * q, isb = sr * q;
+  const double fr = dr * isr, fb = db * isb;
+  const double ur = fr * fr, ub = fb * fb;
+  double rl, rla, rlb, bla, blb, ibl;   // rho_log, partials of both log means, 1/beta_log
+  if (wave_all(ur < TH && ub < TH)) {
+    // l = s/(2F(u)); dl/da = 1/(2F) - l' b, dl/db = 1/(2F) + l' a with
+    // l' = 2 f F'(u) / (s F^2) = 8 F'(u) (f / s) / (2F)^2  (the partials of the series branch)
+    auto partials = [&](double is, double f, double u, double x, double y, double &dx, double &dy) {
+      const double h = logmean_inv_series2<DIM>(u);          // 1/(2F)
+      double Fp8;                                             // 8 F'(u)
+      if constexpr (DIM == 3)
+        Fp8 = 8.0 / 3.0 + u * (16.0 / 5.0 + u * (24.0 / 7.0));
+      else
+        Fp8 = 8.0 / 3.0 + u * (16.0 / 5.0 + u * (24.0 / 7.0 + u * (32.0 / 9.0)));
+      const double t = Fp8 * (f * is) * (h * h);
+      dx = h - t * y;
+      dy = h + t * x;
+      return h;
+    };
+    rl = sr * partials(isr, fr, ur, a.rho, b.rho, rla, rlb);
+    partials(isb, fb, ub, a.beta, b.beta, bla, blb);
+    ibl = isb * logmean_series2<DIM>(ub);                     // 1/bl = 2F(u_beta)/sb
+  } else {
+    double bl;
+    logmean_partials<DIM>(a.rho, b.rho, LAZY_LOGS ? ln(a.rho) : a.lrho, LAZY_LOGS ? ln(b.rho) : b.lrho,
+                          rl, rla, rlb);
+    logmean_partials<DIM>(a.beta, b.beta, LAZY_LOGS ? ln(a.beta) : a.lbeta,
+                          LAZY_LOGS ? ln(b.beta) : b.lbeta, bl, bla, blb);
+    ibl = rcp(bl);
   }
   const double pa = 0.5 * sr * isb;
   double va[DIM], vv = 0.0;
@@ -492,51 +490,54 @@ __device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DI
     va[d] = a.hv[d] + b.hv[d];
     vv = vv + va[d] * va[d];
   }
-  const double vnavg = 2.0 * vv - (a.hq + b.hq);
-  if (!series) ibl = rcp(bl);
-  const double f4 = rl * inv2gm1 * ibl + pa + 0.5 * rl * vnavg;
-  double Un[NT], c0m[NT], A = 0.0, B = 0.0, C = 0.0, tr = 0.0;
+  const double hvn = vv - 0.5 * (a.hq + b.hq);                // vnavg / 2
+  const double gbl = inv2gm1 * ibl;
+  const double rb = rl * gbl;
+  const double f4 = rb + pa + rl * hvn;
+  double Un[NT], c0m[NT], A = 0.0, C = 0.0, tr = 0.0;
   for (int k = 0; k < NT; ++k) {
-    double u = n[k][0] * va[0], cm = c[k][1] * va[0];
+    double u = n[k][0] * va[0], cm = c[k][0] + c[k][1] * va[0];
     for (int d = 1; d < DIM; ++d) {
       u = u + n[k][d] * va[d];
       cm = cm + c[k][1 + d] * va[d];
     }
     for (int d = 0; d < DIM; ++d) tr = tr + n[k][d] * c[k][1 + d];
     Un[k] = u;
-    c0m[k] = c[k][0] + cm;
-    A = A + c[k][0] * u;
-    B = B + u * cm;
+    c0m[k] = cm;
+    A = A + cm * u;                                           // A + B of the comment above
     C = C + c[k][NF - 1] * u;
   }
-  const double L_rl = A + B + C * (inv2gm1 * ibl + 0.5 * vnavg);
-  const double L_bl = -C * rl * inv2gm1 * ibl * ibl;
-  const double L_pa = tr + C;
+  const double L_rl = A + C * (gbl + hvn);
+  const double L_bl = -C * rb * ibl;
+  const double Crl = C * rl;
+  const double hrl = 0.5 * rl, hf4 = 0.5 * f4;
   for (int d = 0; d < DIM; ++d) {
-    double t = 0.0, e = 0.0;
-    for (int k = 0; k < NT; ++k) {
+    // half the derivative by va_d; the |u|^2 terms of the nodes are -Crl u/2 each
+    double t = n[0][d] * c0m[0] + c[0][1 + d] * Un[0];
+    double e = n[0][d] * c[0][NF - 1];
+    for (int k = 1; k < NT; ++k) {
       t = t + n[k][d] * c0m[k] + c[k][1 + d] * Un[k];
       e = e + n[k][d] * c[k][NF - 1];
     }
-    const double L_va = rl * t + f4 * e + C * 2.0 * rl * va[d];
-    const double ua = 2.0 * a.hv[d], ub = 2.0 * b.hv[d];
-    ga.u[d] += 0.5 * L_va - 0.5 * C * rl * ua;
-    gb.u[d] += 0.5 * L_va - 0.5 * C * rl * ub;
+    const double g = hrl * t + hf4 * e + Crl * va[d];
+    ga.u[d] += g - Crl * a.hv[d];
+    gb.u[d] += g - Crl * b.hv[d];
   }
-  ga.rho += L_rl * rla + L_pa * 0.5 * isb;
-  gb.rho += L_rl * rlb + L_pa * 0.5 * isb;
-  ga.beta += L_bl * bla - L_pa * pa * isb;
-  gb.beta += L_bl * blb - L_pa * pa * isb;
+  const double L_pa = (tr + C) * isb;                         // derivative by pa, over sb
+  ga.rho += L_rl * rla + 0.5 * L_pa;
+  gb.rho += L_rl * rlb + 0.5 * L_pa;
+  ga.beta += L_bl * bla - L_pa * pa;
+  gb.beta += L_bl * blb - L_pa * pa;
 }
 
-template <int DIM>
+template <int DIM, bool LAZY_LOGS = false>
 __device__ __forceinline__ void flux_dot_vjp(const Node<DIM> &a, const Node<DIM> &b,
                                              const double (&n)[DIM], const double (&c)[DIM + 2],
                                              double inv2gm1, PrimBar<DIM> &ga, PrimBar<DIM> &gb) {
   double nk[1][DIM], ck[1][DIM + 2];
   for (int d = 0; d < DIM; ++d) nk[0][d] = n[d];
   for (int f = 0; f < DIM + 2; ++f) ck[0][f] = c[f];
-  flux_dot_vjp_k<DIM, 1>(a, b, nk, ck, inv2gm1, ga, gb);
+  flux_dot_vjp_k<DIM, 1, LAZY_LOGS>(a, b, nk, ck, inv2gm1, ga, gb);
 }
 
 // Primitive cotangent -> conservative cotangent of one node:
