@@ -108,6 +108,11 @@ int wadges_update(const wadges_plan *plan, int K, const double *Jq, const double
                   const double *VfPq, double fa, double fb, double fdt, double *rhsQ,
                   double *resQ, double *Q, double *Qf, void *stream);
 
+/* Initial projection of a conservative state (euler.c:4028-4133, on the host in the
+ * reference): rhsQ = u(VqPq v(Q)), Qf = u(VfPq v(Q)), in one launch. */
+int wadges_project(const wadges_plan *plan, int K, const double *VqPq, const double *VfPq,
+                   const double *Q, double *rhsQ, double *Qf, void *stream);
+
 /* One whole LSRK stage in a single launch: vol + surf + update fused per
  * element (no counterpart kernel in the reference; it replaces the three
  * launches of rk_step, euler.c:3656-3666, with one).  The volume RHS stays on

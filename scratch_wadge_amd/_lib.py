@@ -19,7 +19,7 @@ EXPORTED = (
     "wadges_stage", "wadges_stage_record", "wadges_stage_vjp", "wadges_diagnostics",
     "wadges_diagnostics_noalloc",
     "wadges_rhs_vjp", "wadges_update_vjp",
-    "wadges_project_vjp", "wadges_batch_create", "wadges_batch_destroy", "wadges_batch_stage",
+    "wadges_project_vjp", "wadges_project", "wadges_batch_create", "wadges_batch_destroy", "wadges_batch_stage",
     "wadges_batch_run", "wadges_batch_current", "wadges_batch_get_config", "wadges_batch_set_config",
     "wadges_batch_tune",
     "wadges_last_hip_error", "wadges_error_string", "wadges_instance_count", "wadges_instance",
@@ -77,6 +77,7 @@ def load():
     L.wadges_update_vjp.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, ctypes.c_double, ctypes.c_double,
                                     ctypes.c_double] + [_vp] * 6 + [_vp]
     L.wadges_project_vjp.argtypes = [_vp, ctypes.c_int] + [_vp] * 6 + [_vp]
+    L.wadges_project.argtypes = [_vp, ctypes.c_int] + [_vp] * 5 + [_vp]
     L.wadges_batch_create.argtypes = [ctypes.POINTER(_vp), ctypes.c_int, ctypes.c_int,
                                       ctypes.POINTER(Group), ctypes.c_double, ctypes.c_double, _vp]
     L.wadges_batch_destroy.argtypes = [_vp]
@@ -182,6 +183,9 @@ class Plan:
     def project_vjp(self, K, VqPq, VfPq, Q, uq_bar, uf_bar, Q_bar, stream=None):
         check(load().wadges_project_vjp(self.h, K, VqPq, VfPq, Q, uq_bar, uf_bar, Q_bar, stream),
               "wadges_project_vjp")
+
+    def project(self, K, VqPq, VfPq, Q, rhsQ, Qf, stream=None):
+        check(load().wadges_project(self.h, K, VqPq, VfPq, Q, rhsQ, Qf, stream), "wadges_project")
 
     def update(self, K, Jq, VqPq, VfPq, fa, fb, fdt, rhsQ, resQ, Q, Qf, stream=None):
         check(load().wadges_update(self.h, K, Jq, VqPq, VfPq, fa, fb, fdt, rhsQ, resQ, Q, Qf, stream),

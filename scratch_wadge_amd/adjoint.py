@@ -57,19 +57,17 @@ class AdjointSolver:
 
     # ------------------------------------------------------------------ forward
     def _project(self, Q0):
-        """Initial projection rhsQ = u(VqPq v(Q0)), Qf = u(VfPq v(Q0)) on the host
-        side of the driver, like the reference (euler.c:4028-4133)."""
-        prob = self.dev.prob
-        K, nf, Nq = prob.K, prob.nfields, prob.Nq
-        U = Q0.detach().reshape(K, nf, Nq).permute(1, 2, 0)          # (nf, Nq, K)
-        ops = prob.ops
-        VqPq = torch.as_tensor(ops.VqPq, device=U.device)
-        VfPq = torch.as_tensor(ops.VfPq, device=U.device)
-        V = _entropy_vars_t(U, prob.gamma)
-        uq = _conservative_vars_t(torch.einsum("ij,fjk->fik", VqPq, V), prob.gamma)
-        uf = _conservative_vars_t(torch.einsum("ij,fjk->fik", VfPq, V), prob.gamma)
-        lay = lambda X: X.permute(2, 0, 1).contiguous().reshape(-1)
-        return lay(uq), lay(uf)
+        """Initial projection rhsQ = u(VqPq v(Q0)), Qf = u(VfPq v(Q0)) (euler.c:4028-4133)
+        of a float64 state in the Q layout."""
+        d = self.dev
+        if Q0.dtype != torch.float64 or Q0.numel() != d.s["Q"].numel():
+            raise RuntimeError(f"the initial state must hold {d.s['Q'].numel()} float64 values, "
+                               f"got {Q0.numel()} of {Q0.dtype}")
+        Q = Q0.detach().reshape(-1).to(d.device).contiguous()
+        uq, uf = torch.empty_like(d.s["rhsQ"]), torch.empty_like(d.s["Qf"])
+        d.plan.project(d.K, _ptr(d.c["VqPq"]), _ptr(d.c["VfPq"]), _ptr(Q), _ptr(uq), _ptr(uf),
+                       d.stream())
+        return uq, uf
 
     def _set_initial(self, Q0):
         d = self.dev
@@ -189,24 +187,6 @@ class AdjointSolver:
         d.plan.project_vjp(d.K, _ptr(c["VqPq"]), _ptr(c["VfPq"]), _ptr(self.Q0), _ptr(self.uqb),
                            _ptr(self.ufb), _ptr(Qb), d.stream())
         return Qb
-
-
-def _entropy_vars_t(U, gamma):
-    rho, E = U[0], U[-1]
-    m = U[1:-1]
-    rhoe = E - 0.5 * (m * m).sum(0) / rho
-    s = torch.log((gamma - 1.0) * rhoe) - gamma * torch.log(rho)
-    return torch.cat([((-E) / rhoe + (gamma + 1.0 - s))[None], m / rhoe, (-rho / rhoe)[None]], 0)
-
-
-def _conservative_vars_t(V, gamma):
-    vl = V[-1]
-    vv = (V[1:-1] ** 2).sum(0)
-    h = vv / (2.0 * vl)
-    s = gamma - V[0] + h
-    rhoe = torch.exp((torch.log(torch.tensor(gamma - 1.0, dtype=V.dtype, device=V.device))
-                      - gamma * torch.log(-vl) - s) / (gamma - 1.0))
-    return torch.cat([(rhoe * (-vl))[None], rhoe * V[1:-1], (rhoe * (1.0 - h))[None]], 0)
 
 
 class RKRollout(torch.autograd.Function):

@@ -1579,6 +1579,8 @@ struct Ops {
                     const double *, double *, hipStream_t);
   int (*proj_vjp)(const wadges_plan *, int, const double *, const double *, const double *,
                   const double *, const double *, double *, hipStream_t);
+  int (*project)(const wadges_plan *, int, const double *, const double *, const double *,
+                 double *, double *, hipStream_t);
   int (*prep)(const double *, const double *, const double *, const double *, const double *,
               double *, hipStream_t);
   void (*wide)(int, int (&)[2]);
@@ -1850,6 +1852,17 @@ template <class S> int proj_vjp_impl(const wadges_plan *p, int K, const double *
   return hip_check(hipGetLastError());
 }
 
+template <class S> int project_impl(const wadges_plan *p, int K, const double *VqPq,
+                                    const double *VfPq, const double *Q, double *rhsQ, double *Qf,
+                                    hipStream_t st) {
+  if (K == 0) return WADGES_OK;
+  constexpr int TPW = WAVE / S::NQ;
+  constexpr int EPB = 4 * TPW;
+  project_kernel<S, TPW><<<(K + EPB - 1) / EPB, WAVE * 4, 0, st>>>(K, VqPq, VfPq, Q, rhsQ, Qf, p->gamma,
+                                                                  std::log(p->gamma - 1.0));
+  return hip_check(hipGetLastError());
+}
+
 template <class S> int prep_impl(const double *Drq, const double *Dsq, const double *Dtq,
                                  const double *VqLq, const double *VfPq, double *ws,
                                  hipStream_t st) {
@@ -1871,7 +1884,8 @@ template <int DIM, int NQ, int NFQ> constexpr Instance make_instance(int N) {
   return Instance{DIM, N, NQ, NFQ,
                   Ops{&vol_impl<S>, &surf_impl<S>, &update_impl<S>, &stage_impl<S>,
                       &stage_vjp_impl<S>, &diag_impl<S>,
-                      &rhs_vjp_impl<S>, &update_vjp_impl<S>, &proj_vjp_impl<S>, &prep_impl<S>,
+                      &rhs_vjp_impl<S>, &update_vjp_impl<S>, &proj_vjp_impl<S>, &project_impl<S>,
+                      &prep_impl<S>,
                       &wide_limits<S>, S::WS, stage_smem_bytes<S>(), S::TPW}};
 }
 
@@ -2077,6 +2091,13 @@ int wadges_project_vjp(const wadges_plan *p, int K, const double *VqPq, const do
   if (!p || K < 0) return WADGES_EINVAL;
   if (K > 0 && (!VqPq || !VfPq || !Q || !rhsQ_bar || !Qf_bar || !Q_bar)) return WADGES_EINVAL;
   return p->ops.proj_vjp(p, K, VqPq, VfPq, Q, rhsQ_bar, Qf_bar, Q_bar, (hipStream_t)stream);
+}
+
+int wadges_project(const wadges_plan *p, int K, const double *VqPq, const double *VfPq,
+                   const double *Q, double *rhsQ, double *Qf, void *stream) {
+  if (!p || K < 0) return WADGES_EINVAL;
+  if (K > 0 && (!VqPq || !VfPq || !Q || !rhsQ || !Qf)) return WADGES_EINVAL;
+  return p->ops.project(p, K, VqPq, VfPq, Q, rhsQ, Qf, (hipStream_t)stream);
 }
 
 int wadges_stage(const wadges_plan *p, int K, const double *vgeo, const double *vfgeo,

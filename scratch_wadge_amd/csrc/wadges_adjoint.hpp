@@ -659,3 +659,62 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
   }
 }
 
+// Initial projection of a conservative state: u~q = u(VqPq v(Q)), u~f = u(VfPq v(Q))
+// (euler.c:4028-4133).  Bound by its launch on the meshes of one card's adjoint: as
+// tensor operations the same maps were some sixty launches, two operator uploads and
+// 0.65 ms of a 2.44 ms pass (2D N = 3, K = 2,048, two steps and their reverse; now
+// 1.79 ms), 0.6 ms of 4.76 ms at 3D N = 3, K = 10,368 (now 4.17 ms).  Each row has its
+// own lane, the face points of a wave's elements are spread over all of its lanes;
+// the operators (<= 30 KB) come through L1.
+template <class S, int TPW>
+__global__ void __launch_bounds__(WAVE * 4)
+project_kernel(int K, const double *__restrict__ VqPq, const double *__restrict__ VfPq,
+               const double *__restrict__ Q, double *__restrict__ rhsQ, double *__restrict__ Qf,
+               double gamma, double lgm1) {
+  constexpr int DIM = S::DIM, NQ = S::NQ, NFN = S::NFN, NFLD = S::NFLD;
+  constexpr int EPB = 4 * TPW;
+  __shared__ double buf[EPB][NFLD][NQ];
+  const int wave = threadIdx.x / WAVE;
+  const int wl = threadIdx.x % WAVE;
+  const int tw = wl / NQ;
+  const int i = wl - tw * NQ;
+  const bool active = tw < TPW;
+  const int e = wave * TPW + (active ? tw : 0);
+  const int k = blockIdx.x * EPB + e;
+  const bool valid = active && k < K;
+  const size_t base = (valid ? (size_t)k : 0) * NQ * NFLD;
+  if (valid) {
+    double U[NFLD], V[NFLD];
+    for (int f = 0; f < NFLD; ++f) U[f] = Q[base + i + f * NQ];
+    entropy_vars<DIM>(U, gamma, V);
+    for (int f = 0; f < NFLD; ++f) buf[e][f][i] = V[f];
+  }
+  __syncthreads();
+  if (valid) {
+    double U[NFLD], V[NFLD];
+    for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < NQ; ++j) {
+      const double P = ld_off(VqPq, (unsigned)(i + j * NQ));
+      for (int f = 0; f < NFLD; ++f) V[f] += P * buf[e][f][j];
+    }
+    conservative_vars<DIM>(V, gamma, lgm1, U);
+    for (int f = 0; f < NFLD; ++f) rhsQ[base + i + f * NQ] = U[f];
+  }
+  for (int p = wl; p < TPW * NFN; p += WAVE) {
+    const int t = p / NFN;
+    const int fn = p - t * NFN;
+    const int et = wave * TPW + t;
+    const int kt = blockIdx.x * EPB + et;
+    if (kt >= K) continue;
+    double U[NFLD], V[NFLD];
+    for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < NQ; ++j) {
+      const double P = ld_off(VfPq, (unsigned)(fn + j * NFN));
+      for (int f = 0; f < NFLD; ++f) V[f] += P * buf[et][f][j];
+    }
+    conservative_vars<DIM>(V, gamma, lgm1, U);
+    for (int f = 0; f < NFLD; ++f) Qf[(size_t)kt * NFN * NFLD + fn + f * NFN] = U[f];
+  }
+}
