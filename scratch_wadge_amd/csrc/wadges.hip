@@ -1799,11 +1799,8 @@ template <class S> int update_vjp_impl(const wadges_plan *p, int K, const double
                                        const double *uqb, const double *ufb, double *Rb,
                                        hipStream_t st) {
   if (K == 0) return WADGES_OK;
-  constexpr int TPW = WAVE / S::NQ;
-  constexpr int EPB = uvjp_wg_waves<S>() * TPW;
-  update_vjp_kernel<S, TPW><<<(K + EPB - 1) / EPB, WAVE * uvjp_wg_waves<S>(), 0, st>>>(
-      K, Jq, VqPq, VfPq, fa, fb, fdt, Q, Qb, resb, uqb, ufb, Rb, p->gamma, std::log(p->gamma - 1.0),
-      nullptr, nullptr);
+  launch_update_vjp<S>(K, Jq, VqPq, VfPq, fa, fb, fdt, Q, Qb, resb, uqb, ufb, Rb, p->gamma, nullptr,
+                       nullptr, st);
   return hip_check(hipGetLastError());
 }
 
@@ -1825,14 +1822,9 @@ template <class S> int stage_vjp_impl(const wadges_plan *p, int K, const double 
   int rc = ensure_tables<S>(p, Drq, Dsq, Dtq, VqLq, VfPq, st, &tab);
   if (rc) return rc;
   const double g = p->gamma;
-  {
-    constexpr int TPW = WAVE / S::NQ;
-    constexpr int EPB = uvjp_wg_waves<S>() * TPW;
-    update_vjp_kernel<S, TPW><<<(K + EPB - 1) / EPB, WAVE * uvjp_wg_waves<S>(), 0, st>>>(
-        K, Jq, VqPq, VfPq, fa, fb, fdt, Q_out, Qb, resb, uqb_out, ufb_out, Rb, g,
-        std::log(g - 1.0), VqLq, sbar);
-    if ((rc = hip_check(hipGetLastError()))) return rc;
-  }
+  launch_update_vjp<S>(K, Jq, VqPq, VfPq, fa, fb, fdt, Q_out, Qb, resb, uqb_out, ufb_out, Rb, g, VqLq,
+                       sbar, st);
+  if ((rc = hip_check(hipGetLastError()))) return rc;
   constexpr int TPW = WAVE / S::NQ;
   const size_t smem = (size_t)TPW * VjpSmem<S>::per_elem * sizeof(double);
   rhs_vjp_kernel<S, TPW><<<(K + TPW - 1) / TPW, WAVE, smem, st>>>(

@@ -389,16 +389,13 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
 }
 
 // (Q_bar, res_bar) <- stage VJP; R_bar written.  Q is the stage's output state.
-// Workgroup shape of the update VJP.  2D: one wave (its barriers cost nothing),
-// the small operators read through L1.  3D: four waves sharing the operators
-// staged in LDS (the transposed products read them along rows, which through
-// L1 touches a cache line per lane).  3D N = 3 declares three waves per SIMD,
-// as many as its LDS allows (43 KB per four-wave workgroup).
+// Workgroup shape of the update VJPs.  2D: one wave (its barriers cost nothing).  3D:
+// four waves; at N = 1 they share the operators staged in LDS (the transposed products
+// read them along rows, which through L1 touches a cache line per lane).
 template <class S> constexpr int uvjp_wg_waves() { return S::DIM == 2 ? 1 : 4; }
-template <class S> constexpr int update_vjp_waves() { return (S::DIM == 3 && S::NQ == 23) ? 3 : 1; }
 
 template <class S, int TPW>
-__global__ void __launch_bounds__(WAVE * uvjp_wg_waves<S>()) __attribute__((amdgpu_waves_per_eu(update_vjp_waves<S>())))
+__global__ void __launch_bounds__(WAVE * uvjp_wg_waves<S>())
 update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict__ VqPq,
                   const double *__restrict__ VfPq, double fa, double fb, double fdt,
                   const double *__restrict__ Q, double *__restrict__ Qb,
@@ -578,6 +575,212 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
     }
     for (int f = 0; f < NFLD; ++f) sbar[(size_t)kt * NFN * NFLD + f * NFN + fn] = v[f];
   }
+}
+
+// The update VJP with its eight products on MFMA.  A lane per row reads an operator
+// entry and NFLD inputs from LDS for NFLD multiply-adds, and the LDS ports bound the
+// kernel; a 16 x 16 tile reads two values for 16.  The operators come through L1: staged
+// in LDS they cost workgroups per CU and gained nothing.  Bound by the memory it moves
+// and the chain of barriers between the products.  Used where the rows fill enough of a
+// tile: 3D from N = 2, 2D from N = 4.  A pass of two steps and their reverse (four in
+// 2D), a lane per row -> this kernel: 3D N = 2, K = 16,464: 2.32 -> 2.28 ms; N = 3,
+// K = 10,368: 4.15 -> 3.88 ms (update VJP 87 -> 56 us); N = 4, K = 3,072: 3.24 -> 3.10 ms;
+// 2D K = 8,192, N = 4: 1.83 -> 1.74 ms; N = 5: 4.05 -> 3.89 ms.  Below, it loses: 2D
+// N = 1: 0.90 -> 1.03 ms, N = 2: 1.235 -> 1.28 ms, N = 3 (K = 2,048): 1.77 -> 1.80 ms;
+// 3D N = 1: 1.17 -> 1.23 ms.
+template <class S> constexpr bool uvjp_mfma() { return S::DIM == 3 ? S::NQ >= 11 : S::NQ >= 16; }
+
+// OUT[c][i] = sum_j M(i, j) IN[c][j] for the NCOL columns of a workgroup on MFMA, the
+// 16 x 16 tiles spread over its W waves; sums in ascending j, one fused multiply-add
+// per term.  M(i, j) is read through `m` (LDS or L1), IN and OUT are LDS with leading
+// dimensions LDI and LDO.  Columns are independent: those of absent elements hold
+// whatever the LDS held.
+template <int W, int NCOL, int ROWS, int KD, int LDI, int LDO, class M>
+__device__ __forceinline__ void uvjp_product(M m, const double *in, double *out, int lane,
+                                             int wave) {
+  constexpr int MT = (ROWS + 15) / 16, NT = (NCOL + 15) / 16, KS = (KD + 3) / 4;
+  const int lr = lane & 15, lk = lane >> 4;
+  double a[KS];
+  auto load_a = [&](int mt) {
+    const int row = 16 * mt + lr;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int j = 4 * ks + lk;
+      a[ks] = (j < KD && row < ROWS) ? m(row, j) : 0.0;
+    }
+  };
+  constexpr bool FIXED = W % MT == 0;    // a wave's tiles are of one row block
+  if constexpr (FIXED) load_a(wave % MT);
+  for (int t = wave; t < MT * NT; t += W) {
+    const int mt = t % MT;
+    const int c = 16 * (t / MT) + lr;
+    const double *x = in + (c < NCOL ? c : 0) * LDI;
+    double b[KS];
+    if constexpr (!FIXED) load_a(mt);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int j = 4 * ks + lk;
+      b[ks] = j < KD ? x[j] : 0.0;
+    }
+    dbl4 acc = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = mfma_f64_16x16x4(a[ks], b[ks], acc);
+    if (c < NCOL)
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * mt + lk + 4 * r;
+        if (i < ROWS) out[c * LDO + i] = acc[r];
+      }
+  }
+}
+
+template <class S, int TPW>
+__global__ void __launch_bounds__(WAVE * uvjp_wg_waves<S>())
+update_vjp_mfma_kernel(int K, const double *__restrict__ Jq, const double *__restrict__ VqPq,
+                  const double *__restrict__ VfPq, double fa, double fb, double fdt,
+                  const double *__restrict__ Q, double *__restrict__ Qb,
+                  double *__restrict__ resb, const double *__restrict__ uqb,
+                  const double *__restrict__ ufb, double *__restrict__ Rb, double gamma,
+                  double lgm1, const double *__restrict__ VqLq, double *__restrict__ sbar) {
+  constexpr int DIM = S::DIM, NQ = S::NQ, NFN = S::NFN, NFLD = S::NFLD;
+  constexpr int W = uvjp_wg_waves<S>();
+  constexpr int EPB = W * TPW, NCOL = EPB * NFLD;
+  constexpr int LQ = NQ | 1, LF = NFN | 1;     // odd: no bank conflicts across columns
+  __shared__ double bufA[NCOL * LQ];
+  __shared__ double bufB[NCOL * LQ];
+  __shared__ double bufF[NCOL * LF];
+  auto P = [&](int i, int j) { return ld_off(VqPq, (unsigned)(i + j * NQ)); };
+  auto Pt = [&](int i, int j) { return ld_off(VqPq, (unsigned)(j + i * NQ)); };
+  auto Pf = [&](int i, int j) { return ld_off(VfPq, (unsigned)(i + j * NFN)); };
+  auto Pft = [&](int i, int j) { return ld_off(VfPq, (unsigned)(j + i * NFN)); };
+  auto Lt = [&](int i, int j) { return ld_off(VqLq, (unsigned)(j + i * NQ)); };
+  const int wave = threadIdx.x / WAVE;
+  const int wl = threadIdx.x % WAVE;
+  const int tw = wl / NQ;
+  const int i = wl - tw * NQ;
+  const bool active = tw < TPW;
+  const int e = wave * TPW + (active ? tw : 0);
+  const int k = blockIdx.x * EPB + e;
+  const bool valid = active && k < K;
+  const size_t base = (valid ? (size_t)k : 0) * NQ * NFLD;
+  double *A = bufA + e * NFLD * LQ + (active ? i : 0), *B = bufB + e * NFLD * LQ + (active ? i : 0);
+  auto mv = [&](double *in, double *out) {
+    uvjp_product<W, NCOL, NQ, NQ, LQ, LQ>(P, in, out, wl, wave);
+  };
+  auto mvT = [&](double *in, double *out) {
+    uvjp_product<W, NCOL, NQ, NQ, LQ, LQ>(Pt, in, out, wl, wave);
+  };
+
+  double U[NFLD], J = 1.0, invJ = 1.0;
+  if (valid) {
+    J = Jq[(size_t)k * NQ + i];
+    invJ = rcp(J);
+    for (int f = 0; f < NFLD; ++f) U[f] = Q[base + i + f * NQ];
+    double V[NFLD];
+    entropy_vars<DIM>(U, gamma, V);
+    for (int f = 0; f < NFLD; ++f) A[f * LQ] = V[f] * J;
+  }
+  __syncthreads();
+  mv(bufA, bufB);
+  __syncthreads();
+  if (valid)
+    for (int f = 0; f < NFLD; ++f) B[f * LQ] *= invJ;
+  __syncthreads();
+  mv(bufB, bufA);                                    // v~
+  __syncthreads();
+  // cotangents of v~ through u(v~) and u(VfPq v~): the stage writes rhsQ = u(v~)
+  // (v~ already lies in the range of the projection VqPq)
+  uvjp_product<W, NCOL, NFN, NQ, LQ, LF>(Pf, bufA, bufF, wl, wave);
+  double gq[NFLD];
+  if (valid) {
+    double V[NFLD], Ub[NFLD];
+    for (int f = 0; f < NFLD; ++f) V[f] = A[f * LQ];
+    for (int f = 0; f < NFLD; ++f) Ub[f] = uqb[base + i + f * NQ];
+    conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, gq);
+  }
+  __syncthreads();
+  // face points of the wave's TPW elements, spread over all its lanes
+  for (int p = wl; p < TPW * NFN; p += WAVE) {
+    const int t = p / NFN;
+    const int fn = p - t * NFN;
+    const int et = wave * TPW + t;
+    const int kt = blockIdx.x * EPB + et;
+    if (kt >= K) continue;
+    double *F = bufF + et * NFLD * LF + fn;
+    double V[NFLD], Ub[NFLD], g[NFLD];
+    for (int f = 0; f < NFLD; ++f) V[f] = F[f * LF];
+    for (int f = 0; f < NFLD; ++f) Ub[f] = ufb[(size_t)kt * NFN * NFLD + fn + f * NFN];
+    conservative_vars_vjp<DIM>(V, gamma, lgm1, Ub, g);
+    for (int f = 0; f < NFLD; ++f) F[f * LF] = g[f];
+  }
+  __syncthreads();
+  // v~_bar = g_q + VfPq^T g_f ; then through VqPq diag(1/J) VqPq
+  uvjp_product<W, NCOL, NQ, NFN, LF, LQ>(Pft, bufF, bufB, wl, wave);
+  __syncthreads();
+  if (valid)
+    for (int f = 0; f < NFLD; ++f) B[f * LQ] += gq[f];
+  __syncthreads();
+  mvT(bufB, bufA);
+  __syncthreads();
+  if (valid)
+    for (int f = 0; f < NFLD; ++f) A[f * LQ] *= invJ;
+  __syncthreads();
+  mvT(bufA, bufB);
+  __syncthreads();
+  if (valid) {
+    double Vb[NFLD], Ub[NFLD];
+    for (int f = 0; f < NFLD; ++f) Vb[f] = J * B[f * LQ];
+    entropy_vars_vjp<DIM>(U, gamma, Vb, Ub);
+    for (int f = 0; f < NFLD; ++f) {
+      const size_t id = base + i + f * NQ;
+      const double qb = Qb[id] + Ub[f];        // cotangent of Q'
+      const double resb_tot = resb[id] + fb * qb;  // Q' = Q + fb res'
+      Qb[id] = qb;
+      resb[id] = fa * resb_tot;
+      A[f * LQ] = fdt * resb_tot;              // r_bar
+    }
+  }
+  // R_bar = -2 VqPq^T diag(1/J) VqPq^T r_bar
+  __syncthreads();
+  mvT(bufA, bufB);
+  __syncthreads();
+  if (valid)
+    for (int f = 0; f < NFLD; ++f) B[f * LQ] *= invJ;
+  __syncthreads();
+  mvT(bufB, bufA);
+  __syncthreads();
+  if (valid)
+    for (int f = 0; f < NFLD; ++f) {
+      const double rbar = -2.0 * A[f * LQ];
+      Rb[base + i + f * NQ] = rbar;
+      A[f * LQ] = rbar;
+    }
+  if (!sbar) return;  // uniform: a kernel argument
+  // s_bar = VqLq^T R_bar at this element's face points (what sbar_kernel computes)
+  __syncthreads();
+  uvjp_product<W, NCOL, NFN, NQ, LQ, LF>(Lt, bufA, bufF, wl, wave);
+  __syncthreads();
+  for (int p = threadIdx.x; p < NCOL * NFN; p += WAVE * W) {
+    const int c = p / NFN;
+    const size_t at = (size_t)blockIdx.x * NCOL * NFN + p;
+    if ((int)blockIdx.x * EPB + c / NFLD < K) sbar[at] = bufF[c * LF + p - c * NFN];
+  }
+}
+
+template <class S>
+inline void launch_update_vjp(int K, const double *Jq, const double *VqPq, const double *VfPq,
+                              double fa, double fb, double fdt, const double *Q, double *Qb,
+                              double *resb, const double *uqb, const double *ufb, double *Rb,
+                              double gamma, const double *VqLq, double *sbar, hipStream_t st) {
+  constexpr int TPW = WAVE / S::NQ, T = WAVE * uvjp_wg_waves<S>();
+  constexpr int EPB = uvjp_wg_waves<S>() * TPW;
+  const int blocks = (K + EPB - 1) / EPB;
+  const double lgm1 = std::log(gamma - 1.0);
+  if constexpr (uvjp_mfma<S>())
+    update_vjp_mfma_kernel<S, TPW><<<blocks, T, 0, st>>>(K, Jq, VqPq, VfPq, fa, fb, fdt, Q, Qb, resb, uqb,
+                                                         ufb, Rb, gamma, lgm1, VqLq, sbar);
+  else
+    update_vjp_kernel<S, TPW><<<blocks, T, 0, st>>>(K, Jq, VqPq, VfPq, fa, fb, fdt, Q, Qb, resb, uqb,
+                                                    ufb, Rb, gamma, lgm1, VqLq, sbar);
 }
 
 // Q_bar += VJP of (u~q, u~f) = (u(VqPq v(Q)), u(VfPq v(Q))) at Q.
