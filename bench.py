@@ -272,7 +272,7 @@ def vjp_kernel_times(dev, adj, reps=5):
         torch.cuda.synchronize()
         ms = float(np.mean([a.elapsed_time(b) for a, b in evs]))
         entry = {"launch_ms": round(ms, 4)}
-        kern = {"stage_record": "stage_kernel", "update_vjp": "update_vjp_kernel",
+        kern = {"stage_record": "team_stage_kernel", "update_vjp": "update_vjp_mfma_kernel",
                 "rhs_vjp": "rhs_vjp_kernel"}[name]
         fl = prof("fp64_lane_flops_per_launch", kern)
         if fl is not None:
@@ -439,6 +439,10 @@ def main():
                  f"_K{prob.K}_N{prob.N}.md")
     prof = lambda key, kernel: profiled_value(key, kernel, prof_file)
 
+    # 3D N = 3 runs a wave per face, the other shapes a team of lanes per element
+    team = "team_" if (prob.dim, prob.N) == (3, 3) else ""
+    stage_kernel, vol_kernel = team + "stage_kernel", team + "vol_kernel"
+
     def counter_tflops(kernel, ms):
         v = prof("fp64_lane_flops_per_launch", kernel)
         return None if v is None else round(v / (ms * 1e-3) / 1e12, 3)
@@ -498,28 +502,28 @@ def main():
                     "elementwise D o F over node pairs, not a matrix product; the "
                     "small dense operator products (lift, VqPq, face traces) run on "
                     "the FP64 matrix cores, whose dense peak equals the vector peak",
-            "kernel": "stage_kernel",
+            "kernel": stage_kernel,
             "achieved": round(achieved, 3), "peak": W.FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(achieved / W.FP64_PEAK_TFLOPS, 4),
             "flops_per_launch": flops,
             "flops_per_element": W.stage_flops(prob.dim, prob.Nq, prob.Nf),
             "launch_ms": round(stage_ms, 4),
-            "traffic": prof("traffic_bytes_per_launch", "stage_kernel"),
+            "traffic": prof("traffic_bytes_per_launch", stage_kernel),
             "traffic_source": "rocprofv3 FETCH_SIZE x2.0 + WRITE_SIZE x1.0 (copy-calibrated), "
                               f"profiles/{prof_file}",
-            "counter_tflops": counter_tflops("stage_kernel", stage_ms),
+            "counter_tflops": counter_tflops(stage_kernel, stage_ms),
             "counter_source": "64 (ADD+MUL+TRANS) + 128 FMA FP64 instructions per launch "
                               f"(SQ_INSTS_VALU_*_F64), profiles/{prof_file}, over launch_ms; "
                               "vector ALU only, the matrix-core products are not in these counters",
-            "profile_kernel_avg_ms": prof_ms("stage_kernel"),
+            "profile_kernel_avg_ms": prof_ms(stage_kernel),
         },
-        "vol_kernel_roofline": {"bound": "fp64 valu", "kernel": "vol_kernel",
+        "vol_kernel_roofline": {"bound": "fp64 valu", "kernel": vol_kernel,
                                 "achieved": round(vflops / (vol_ms * 1e-3) / 1e12, 3),
                                 "frac": round(vflops / (vol_ms * 1e-3) / 1e12 / W.FP64_PEAK_TFLOPS, 4),
                                 "flops_per_element": W.vol_flops(prob.dim, prob.Nq, prob.Nf),
                                 "launch_ms": round(vol_ms, 4),
-                                "counter_tflops": counter_tflops("vol_kernel", vol_ms),
-                                "profile_kernel_avg_ms": prof_ms("vol_kernel")},
+                                "counter_tflops": counter_tflops(vol_kernel, vol_ms),
+                                "profile_kernel_avg_ms": prof_ms(vol_kernel)},
         "hbm_GBs": {
             "stage_fused": round(W.bytes_stage_fused(prob.dim, prob.Nq, prob.Nf) * prob.K / (stage_ms * 1e-3) / 1e9, 1),
             "surf": round(W.bytes_surf(prob.dim, prob.Nq, prob.Nf) * prob.K / (surf_ms * 1e-3) / 1e9, 1),

@@ -21,6 +21,12 @@
 //                  entropy projection and u(v) at volume and face points.
 //                  HBM / transcendental bound; operators staged in LDS.
 //
+// and the fused stage, one launch for all three, in three forms that give the same
+// bits: stage_kernel (a team of lanes per element, ensembles too), team_stage_kernel
+// (3D N = 3: a wave per face, wadges_team.hpp; team_vol_kernel is its volume part) and
+// stage_wide (launches that fit the card at once: an element's pairs over a workgroup,
+// wadges_wide.hpp).
+//
 // Operator tables of vol_kernel are re-laid out per call by a tiny prep kernel
 // into the plan's workspace, "diagonal-major": entry [t][i] belongs to the pair
 // (i, (i + t) mod L), so at step t the lanes of every team read consecutive
