@@ -336,6 +336,10 @@ __device__ __forceinline__ void store_node(double *rec, int stride, int j, const
   rec[(DIM + 4) * stride + j] = n.hq;
 }
 
+// LDS written by lanes of this wave is read by others of it: LDS operations of a
+// wave keep their order, the fence keeps the compiler's.
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
 // Where the other teams of the wave find their data (for phases that spread the
 // face points of all elements of a wave over all 64 lanes).
 struct WaveCtx {
@@ -358,7 +362,8 @@ struct WaveCtx {
 // (rhsQf).  Uq is the element's projected
 // volume state, vg its volume geofacs; the face state and geofacs of the wave's
 // elements come through wc.  Every lane of the workgroup must call this
-// (barriers).
+// (barriers: none under a condition that two waves of a workgroup may answer
+// differently, since ensembles run workgroups of several waves).
 template <class S>
 __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, const double *vg,
                                          const double (*s_nref)[S::DIM], const double *ws,
@@ -417,7 +422,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
       vrec[(DIM + 2) * NQ + l + r * LPE] = me[r].lrho;
       vrec[(DIM + 3) * NQ + l + r * LPE] = me[r].lbeta;
     }
-    __syncthreads();
+    wave_fence();   // read by this wave only; others of the workgroup may be smooth
   }
 
   for (int r = 0; r < R; ++r)
@@ -683,7 +688,7 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
         frect[(DIM + 2) * NH + fl] = ln(frect[0 * NH + fl]);
         frect[(DIM + 3) * NH + fl] = ln(frect[(DIM + 1) * NH + fl]);
       }
-      __syncthreads();
+      wave_fence();   // read by this wave only; others of the workgroup may be smooth
     }
     if (valid) {
       if constexpr (R > 1) {

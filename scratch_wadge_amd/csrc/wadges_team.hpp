@@ -58,10 +58,6 @@ template <class S> struct TeamLane {
   }
 };
 
-// LDS written by lanes of this wave is read by others of it: LDS operations of a
-// wave keep their order, the fence keeps the compiler's.
-__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
 // Volume term of the workgroup's elements.  On return LDS holds, per element, the
 // volume accumulators T_w of the waves from 0 on, the row sums P_w of face w at the
 // start of that face's record block, and the face rows (rhsQf) at AFOFF (this wave's
