@@ -262,7 +262,9 @@ __device__ __forceinline__ bool in_smooth_band(double rho, double beta, double r
 // the log branches (same bits).  In the 2D pair loops the test does not pay: the
 // kernels aim at four or more waves per SIMD and spilled with it.  LAZY_LOGS: the
 // nodes come without logarithms, which are taken only behind that test (the
-// surface flux, whose two nodes serve one pair).
+// surface flux, whose two nodes serve one pair).  Differences of logarithms there
+// too, not the logarithm of a quotient: they change sign exactly when the nodes
+// change places, so the two elements of a face take the same flux.
 // smooth: a wave-uniform flag by which the caller guarantees (3D) that every
 // active lane's pair takes the series branch of both log means; the per-pair
 // wave test is then skipped (the same branch, so the same bits).
@@ -285,8 +287,8 @@ __device__ __forceinline__ PairFlux<DIM> pair_flux(const Node<DIM> &a, const Nod
   const bool all_series = (DIM == 3 || LAZY_LOGS) && (smooth || wave_all(serR && serB));
   if (!all_series) {
     // rho_log = dr / (ln rho_a - ln rho_b), 1/beta_log = (ln beta_a - ln beta_b) / db
-    const double ldR = LAZY_LOGS ? ln(a.rho * rcp(b.rho)) : a.lrho - b.lrho;
-    const double ldB = LAZY_LOGS ? ln(a.beta * rcp(b.beta)) : a.lbeta - b.lbeta;
+    const double ldR = LAZY_LOGS ? ln(a.rho) - ln(b.rho) : a.lrho - b.lrho;
+    const double ldB = LAZY_LOGS ? ln(a.beta) - ln(b.beta) : a.lbeta - b.lbeta;
     const double dR = serR ? 1.0 : ldR;
     const double dB = serB ? 1.0 : db;
     const double q2 = rcp(dR * dB);
