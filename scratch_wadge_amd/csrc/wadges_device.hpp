@@ -44,6 +44,8 @@ template <int DIM> struct Node {
 // arguments) and one third-order step, r (1 + e + e^2) with e = 1 - x r: the
 // omitted e^3 is below 2^-72.  The same results as two Newton steps (at most half
 // an ulp off on those arguments) in three multiply-adds instead of four.
+// For arguments whose reciprocal is a normal number; 0, infinities and subnormal
+// arguments give NaN (IEEE division: infinity and 0).  No admissible state has them.
 __device__ __forceinline__ double rcp(double x) {
   const double r = __builtin_amdgcn_rcp(x);
   const double e = __builtin_fma(-x, r, 1.0);
@@ -51,7 +53,8 @@ __device__ __forceinline__ double rcp(double x) {
 }
 
 // a/b given r = rcp(b): one correction of the quotient by its remainder (within
-// 0.51 ulp for normal operands) instead of the scaled IEEE sequence.
+// 0.51 ulp for normal operands and quotients) instead of the scaled IEEE sequence.
+// NaN where rcp(b) is, and for an infinite a.
 __device__ __forceinline__ double quot(double a, double b, double r) {
   const double q = a * r;
   return __builtin_fma(__builtin_fma(-b, q, a), r, q);
@@ -63,7 +66,9 @@ __device__ __forceinline__ double quot(double a, double b, double r) {
 // accurate: against 80-bit arithmetic over 4M arguments each, rms error ln 0.289
 // ulp (library 0.289-0.293; arguments in [1/2, 2], [1e-6, 1e6], [1e-300, 1e300]),
 // expo 0.302 (0.302; [-8, 8], [-700, 700]), root 0.289 (0.289).  Arguments outside
-// their domain give what the library gives (NaN, infinities, zero).  With them and
+// their domain give what the library gives (NaN, infinities, zero), but for ln of a
+// negative number that rounds to -0 in single precision: -infinity (which quot() turns
+// into NaN in the maps to conservative variables).  With them and
 // quot() in place of IEEE division: 2D N = 4, K = 32,258, a step 434 -> 397 us; the
 // 64-problem ensemble 3.11 -> 2.83 ms for two steps; 3D N = 3, K = 196,608, 8.9 ->
 // 8.75 ms.
@@ -79,6 +84,9 @@ __device__ __forceinline__ double sconst(double v) {
 constexpr double LN2_HI = 0x1.62e42fefp-1;           // 32 bits: k LN2_HI is exact, |k| < 2^20
 constexpr double LN2_LO = 0x1.473de6af278edp-34;     // ln 2 - LN2_HI
 
+// The arrangement of ln is that of fdlibm's log (f and f^2/2 kept out of the rounded
+// part, the series in two interleaved chains), with the Taylor coefficients of atanh.
+//
 // ln x: x = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact), s = f/(2+f)
 // and ln(1+f) = 2 atanh(s) = f - f^2/2 + s (f^2/2 + R(s^2)) with R(z) = 2 (z/3 +
 // z^2/5 + ...) (s f = f^2/2 - s f^2/2 ... regroups the first term so that f enters
