@@ -76,6 +76,11 @@ int wadges_plan_create(wadges_plan **plan, int dim, int N, int Nq, int Nfq, doub
 int wadges_plan_destroy(wadges_plan *plan);
 /* Forgets the prepared operator tables (see above); the next call prepares them. */
 int wadges_plan_invalidate(wadges_plan *plan);
+/* The largest K whose fused stage takes the launch of up to two elements per CU
+ * (*small) and the larger one that fills the device once (*large); meshes beyond
+ * take the packed stage.  Both 0 where the shape has one fused launch for every K.
+ * Found from the device's occupancy at plan creation, which fails if that query does. */
+int wadges_plan_wide_limits(const wadges_plan *plan, int *small, int *large);
 
 /* Volume kernel: role of euler_vol_3d_curved (okl/Euler3D.okl:2123-2523),
  * euler_vol_2d_curved (okl/Euler2D.okl:773-1353) and, on affine meshes, of

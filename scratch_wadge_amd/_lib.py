@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(HERE, "libwadges.so")
 
 # Every symbol the header declares (checked by the CPU tests).
 EXPORTED = (
-    "wadges_plan_create", "wadges_plan_destroy", "wadges_plan_invalidate", "wadges_vol", "wadges_surf", "wadges_update",
+    "wadges_plan_create", "wadges_plan_destroy", "wadges_plan_invalidate", "wadges_plan_wide_limits", "wadges_vol", "wadges_surf", "wadges_update",
     "wadges_stage", "wadges_stage_record", "wadges_stage_vjp", "wadges_diagnostics",
     "wadges_diagnostics_noalloc",
     "wadges_rhs_vjp", "wadges_update_vjp",
@@ -62,6 +62,7 @@ def load():
                                      ctypes.c_int, ctypes.c_double, ctypes.c_double]
     L.wadges_plan_destroy.argtypes = [_vp]
     L.wadges_plan_invalidate.argtypes = [_vp]
+    L.wadges_plan_wide_limits.argtypes = [_vp] + [ctypes.POINTER(ctypes.c_int)] * 2
     L.wadges_vol.argtypes = [_vp, ctypes.c_int] + [_vp] * 15 + [_vp]
     L.wadges_surf.argtypes = [_vp, ctypes.c_int] + [_vp] * 6 + [_vp]
     L.wadges_update.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, ctypes.c_double, ctypes.c_double,
@@ -134,6 +135,13 @@ class Plan:
 
     def invalidate(self):
         check(load().wadges_plan_invalidate(self.h), "wadges_plan_invalidate")
+
+    def wide_limits(self):
+        """Largest K of the fused stage's two launches for small meshes."""
+        a, b = ctypes.c_int(), ctypes.c_int()
+        check(load().wadges_plan_wide_limits(self.h, ctypes.byref(a), ctypes.byref(b)),
+              "wadges_plan_wide_limits")
+        return a.value, b.value
 
     def vol(self, K, vgeo, vfgeo, nrJ, nsJ, ntJ, Drq, Dsq, Dtq, Drstq, VqLq, VfPq, Q, Qf, rhsQ,
             rhsQf, stream=None):

@@ -1597,7 +1597,7 @@ struct Ops {
                  double *, double *, hipStream_t);
   int (*prep)(const double *, const double *, const double *, const double *, const double *,
               double *, hipStream_t);
-  void (*wide)(int, int (&)[2]);
+  int (*wide)(int, int (&)[2]);
   int ws_doubles;
   int stage_smem;  // dynamic LDS bytes of one fused-stage workgroup
   int stage_tpw;   // elements per fused-stage workgroup
@@ -1751,19 +1751,22 @@ template <class S> int stage_impl(const wadges_plan *p, int K, const double *vge
 }
 
 // Largest meshes of the two wide launches on a device of `cus` CUs (0: none).
-template <class S> void wide_limits(int cus, int (&k)[2]) {
+template <class S> int wide_limits(int cus, int (&k)[2]) {
   k[0] = k[1] = 0;
   if constexpr (S::R == 1) {
     using Small = typename WideChoice<S>::Small;
     using Large = typename WideChoice<S>::Large;
-    int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Small>, Small::T,
-                                                     Small::bytes) == hipSuccess)
-      k[0] = std::min(2, occ * Small::E) * cus;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_wide<Large>, Large::T,
-                                                     Large::bytes) == hipSuccess)
-      k[1] = occ * Large::E * cus;
+    int small = 0, large = 0;
+    int rc = hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&small, stage_wide<Small>,
+                                                                    Small::T, Small::bytes));
+    if (!rc)
+      rc = hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&large, stage_wide<Large>,
+                                                                  Large::T, Large::bytes));
+    if (rc) return rc;
+    k[0] = std::min(2, small * Small::E) * cus;
+    k[1] = large * Large::E * cus;
   }
+  return WADGES_OK;
 }
 
 template <class S> int diag_impl(const wadges_plan *p, int K, const double *wq, const double *Jq,
@@ -1970,10 +1973,14 @@ int wadges_plan_create(wadges_plan **plan, int dim, int N, int Nq, int Nfq, doub
     delete p;
     return WADGES_EHIP;
   }
-  p->wide_k[0] = p->wide_k[1] = 0;
   int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess)
-    inst->ops.wide(cus, p->wide_k);
+  int rc = hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device));
+  if (!rc) rc = inst->ops.wide(cus, p->wide_k);
+  if (rc) {
+    (void)hipGetLastError();      // reported here, not by the next launch
+    delete p;
+    return rc;
+  }
   // the fixed diagnostics array of this device (looked up once per device; a
   // failure here is reported by wadges_diagnostics_noalloc, which retries)
   p->scratch_addr = nullptr;
@@ -1994,6 +2001,13 @@ int wadges_plan_destroy(wadges_plan *plan) {
   if (plan->ws) rc = hip_check(hipFree(plan->ws));
   delete plan;
   return rc;
+}
+
+int wadges_plan_wide_limits(const wadges_plan *plan, int *small, int *large) {
+  if (!plan || !small || !large) return WADGES_EINVAL;
+  *small = plan->wide_k[0];
+  *large = plan->wide_k[1];
+  return WADGES_OK;
 }
 
 int wadges_plan_invalidate(wadges_plan *plan) {
