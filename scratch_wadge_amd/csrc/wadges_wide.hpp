@@ -139,8 +139,8 @@ __device__ __forceinline__ void wide_product(const TileA<W, ROWS, KD> &A, int in
   }
 }
 
-// Two waves per SIMD declared: 128 or 168 registers spill (the batched LDS reads of
-// the sums), and a launch that fills more goes to the packed stage.
+// Two waves per SIMD declared: 128 or 168 registers spill in several shapes (the batched
+// LDS reads of the sums), and a launch that fills more goes to the packed stage.
 template <class X>
 __global__ void __launch_bounds__(X::T) __attribute__((amdgpu_waves_per_eu(2)))
 stage_wide(StageArgs args) {
@@ -435,7 +435,10 @@ stage_wide(StageArgs args) {
         constexpr int GR = face_groups<S>(), FH = Vf::FH;
         static_assert(CF == Vf::STEPS, "whole walk at a time");
         const int h = face / FH, fh = face - h * FH;
-#pragma unroll
+        // 3D N = 2: with the sums of both faces of a part in flight the kernel spilled
+        // (28 bytes a lane; a stage at K = 162, 750 and 1,000 13.7, 16.0 and 17.1 us,
+        // one face at a time 13.2, 15.3 and 16.5)
+#pragma unroll (DIM == 3 && NQ == 11 ? 1 : FH)
         for (int u = 0; u < FH; ++u) {
           int g0 = fh - u;
           if (g0 < 0) g0 += FH;
