@@ -148,9 +148,10 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
     __syncthreads();
   }
   // Loops kept rolled where unrolled completely they spill or leave one wave per SIMD
-  // (3D N = 1, 2; 2D from N = 3 on): 3D N = 2, K = 16,464, 101 -> 81 us; 2D N = 4, K =
-  // 8,192, 36 -> 30 us.  The other shapes lose 5 % by it.
-  constexpr bool ROLLED = DIM == 3 ? NQ <= 11 : NQ >= 12;
+  // (3D N = 1, 2; 2D from N = 2 on): 3D N = 2, K = 16,464, 101 -> 81 us; 2D N = 4, K =
+  // 8,192, 36 -> 30 us; 2D N = 2, K = 12,288 and 32,768, 39 -> 29 and 65 -> 50 us (8,192
+  // and less the same).  The other shapes lose 5 % by it.
+  constexpr bool ROLLED = DIM == 3 ? NQ <= 11 : NQ >= 6;
   auto bound = [](int v) { return ROLLED ? opaque_bound(v) : v; };
   if (valid) {
     const double *Dfw = ws;
