@@ -314,8 +314,8 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
       sbM[f] = sbt[f * NFN + fn];
       cons[f] = 0.0;
     }
-    const Node<DIM> a = make_node<DIM, false>(UM, gm1);
-    const Node<DIM> b = make_node<DIM, false>(UP, gm1);
+    Node<DIM> a = make_node<DIM, false>(UM, gm1);
+    Node<DIM> b = make_node<DIM, false>(UP, gm1);
     double hnM[DIM];
     for (int d = 0; d < DIM; ++d) hnM[d] = 0.5 * g[fn + d * NFN];
     const double sJM = g[fn + DIM * NFN];
@@ -349,7 +349,7 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
       for (int f = 0; f < NFLD; ++f) sbP[f] = sbar[idP + (size_t)f * NFN];
       PrimBar<DIM> gx;
       primbar_zero<DIM>(gx);
-      flux_dot_vjp<DIM, true>(b, a, hnP, sbP, inv2gm1, gx, ga);
+      flux_dot_vjp<DIM>(b, a, hnP, sbP, inv2gm1, gx, ga);   // logarithms: taken above if needed
       const double LfP = ltau * fmax(lamP, lamM) * sJP;
       double S2 = 0.0;
       for (int f = 0; f < NFLD; ++f) S2 = S2 + sbP[f] * (UM[f] - UP[f]);

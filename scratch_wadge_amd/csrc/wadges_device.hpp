@@ -451,10 +451,11 @@ __device__ __forceinline__ void logmean_partials(double a, double b, double la, 
 //
 // When every active lane of the wave takes the series branch of both log means
 // (smooth states), 1/F comes from the series of 1/F and every reciprocal of the pair
-// from one.  LAZY_LOGS: the nodes come without logarithms, which are then taken only
-// behind that test (the surface flux, whose nodes serve one pair per side).
-template <int DIM, int NT, bool LAZY_LOGS = false>
-__device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DIM> &b,
+// from one.  LAZY_LOGS: the nodes come without logarithms, which are taken only behind
+// that test and kept in them (the surface flux, whose second pair of the same nodes runs
+// on some of the first one's lanes and so needs them only if the first did).
+template <int DIM, int NT, bool LAZY_LOGS = false, class NA, class NB>
+__device__ __forceinline__ void flux_dot_vjp_k(NA &a, NB &b,
                                                const double (&n)[NT][DIM],
                                                const double (&c)[NT][DIM + 2], double inv2gm1,
                                                PrimBar<DIM> &ga, PrimBar<DIM> &gb) {
@@ -488,10 +489,14 @@ __device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DI
     ibl = isb * logmean_series2<DIM>(ub);                     // 1/bl = 2F(u_beta)/sb
   } else {
     double bl;
-    logmean_partials<DIM>(a.rho, b.rho, LAZY_LOGS ? ln(a.rho) : a.lrho, LAZY_LOGS ? ln(b.rho) : b.lrho,
-                          rl, rla, rlb);
-    logmean_partials<DIM>(a.beta, b.beta, LAZY_LOGS ? ln(a.beta) : a.lbeta,
-                          LAZY_LOGS ? ln(b.beta) : b.lbeta, bl, bla, blb);
+    if constexpr (LAZY_LOGS) {
+      a.lrho = ln(a.rho);
+      a.lbeta = ln(a.beta);
+      b.lrho = ln(b.rho);
+      b.lbeta = ln(b.beta);
+    }
+    logmean_partials<DIM>(a.rho, b.rho, a.lrho, b.lrho, rl, rla, rlb);
+    logmean_partials<DIM>(a.beta, b.beta, a.lbeta, b.lbeta, bl, bla, blb);
     ibl = rcp(bl);
   }
   const double pa = 0.5 * sr * isb;
@@ -540,8 +545,8 @@ __device__ __forceinline__ void flux_dot_vjp_k(const Node<DIM> &a, const Node<DI
   gb.beta += L_bl * blb - L_pa * pa;
 }
 
-template <int DIM, bool LAZY_LOGS = false>
-__device__ __forceinline__ void flux_dot_vjp(const Node<DIM> &a, const Node<DIM> &b,
+template <int DIM, bool LAZY_LOGS = false, class NA, class NB>
+__device__ __forceinline__ void flux_dot_vjp(NA &a, NB &b,
                                              const double (&n)[DIM], const double (&c)[DIM + 2],
                                              double inv2gm1, PrimBar<DIM> &ga, PrimBar<DIM> &gb) {
   double nk[1][DIM], ck[1][DIM + 2];
