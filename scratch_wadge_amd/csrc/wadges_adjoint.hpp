@@ -394,6 +394,12 @@ rhs_vjp_kernel(int K, const double *__restrict__ vgeo, const double *__restrict_
 // four waves; at N = 1 they share the operators staged in LDS (the transposed products
 // read them along rows, which through L1 touches a cache line per lane).
 template <class S> constexpr int uvjp_wg_waves() { return S::DIM == 2 ? 1 : 4; }
+// Whether the products next to the nonlinear maps, in these kernels and in
+// proj_vjp_kernel, are unrolled completely.  In parts elsewhere: completely, the larger
+// shapes spill and 2D N = 3 to 5 lose waves (4 to 10 % at K >= 12,288).  2D N = 2, K =
+// 2,048, four at a time / completely: update VJP 9.3 / 8.6 us, projection VJP 8.9 / 7.9;
+// 3D N = 1: projection VJP 8.5 / 8.2; 2D N = 5, four / eight at a time: 12.0 / 10.8.
+template <class S> constexpr bool vjp_unrolled() { return S::NQ <= 6; }
 
 template <class S, int TPW>
 __global__ void __launch_bounds__(WAVE * uvjp_wg_waves<S>())
@@ -407,6 +413,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
   constexpr int WPB = uvjp_wg_waves<S>();
   constexpr bool OPS_LDS = WPB > 1;
   constexpr int EPB = WPB * TPW;
+  constexpr int UNROLL = vjp_unrolled<S>() ? NQ : 4, UNROLLF = vjp_unrolled<S>() ? NFN : 8;
   __shared__ double sP[OPS_LDS ? NQ * NQ : 1];
   __shared__ double sPf[OPS_LDS ? NFN * NQ : 1];
   __shared__ double bufA[EPB][NFLD][NQ];
@@ -492,7 +499,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
     if (kt >= K) continue;
     double V[NFLD], Ub[NFLD], g[NFLD];
     for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int j = 0; j < NQ; ++j) {
       const double P = Pf(fn + j * NFN);
       for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[et][f][j];
@@ -506,7 +513,7 @@ update_vjp_kernel(int K, const double *__restrict__ Jq, const double *__restrict
   if (valid) {
     double r[NFLD];
     for (int f = 0; f < NFLD; ++f) r[f] = bufB[e][f][i];
-#pragma unroll 8
+#pragma unroll UNROLLF
     for (int fn = 0; fn < NFN; ++fn) {
       const double P = Pf(fn + i * NFN);
       for (int f = 0; f < NFLD; ++f) r[f] += P * bufF[e][f][fn];
@@ -793,6 +800,8 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
                 double lgm1) {
   constexpr int DIM = S::DIM, NQ = S::NQ, NFN = S::NFN, NFLD = S::NFLD;
   constexpr int EPB = 4 * TPW;
+  constexpr int PART = DIM == 2 && NQ >= 16 ? 8 : 4;
+  constexpr int UNROLL = vjp_unrolled<S>() ? NQ : PART, UNROLLF = vjp_unrolled<S>() ? NFN : PART;
   __shared__ double bufA[EPB][NFLD][NQ];
   __shared__ double bufB[EPB][NFLD][NQ];
   __shared__ double bufF[EPB][NFLD][NFN];
@@ -818,7 +827,7 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
   if (valid) {
     double V[NFLD], Ub[NFLD], g[NFLD];
     for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int j = 0; j < NQ; ++j) {
       const double P = ld_off(VqPq, (unsigned)(i + j * NQ));
       for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[e][f][j];
@@ -835,7 +844,7 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
     if (kt >= K) continue;
     double V[NFLD], Ub[NFLD], g[NFLD];
     for (int f = 0; f < NFLD; ++f) V[f] = 0.0;
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int j = 0; j < NQ; ++j) {
       const double P = ld_off(VfPq, (unsigned)(fn + j * NFN));
       for (int f = 0; f < NFLD; ++f) V[f] += P * bufA[et][f][j];
@@ -848,12 +857,12 @@ proj_vjp_kernel(int K, const double *__restrict__ VqPq, const double *__restrict
   if (valid) {
     double vb[NFLD], Ub[NFLD];
     for (int f = 0; f < NFLD; ++f) vb[f] = 0.0;
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int j = 0; j < NQ; ++j) {
       const double P = ld_off(VqPq, (unsigned)(j + i * NQ));
       for (int f = 0; f < NFLD; ++f) vb[f] += P * bufB[e][f][j];
     }
-#pragma unroll 4
+#pragma unroll UNROLLF
     for (int fn = 0; fn < NFN; ++fn) {
       const double P = ld_off(VfPq, (unsigned)(fn + i * NFN));
       for (int f = 0; f < NFLD; ++f) vb[f] += P * bufF[e][f][fn];
