@@ -295,8 +295,10 @@ __device__ __forceinline__ PairFlux<DIM> pair_flux(const Node<DIM> &a, const Nod
   const bool all_series = (DIM == 3 || LAZY_LOGS) && (smooth || wave_all(serR && serB));
   if (!all_series) {
     // rho_log = dr / (ln rho_a - ln rho_b), 1/beta_log = (ln beta_a - ln beta_b) / db
+    double ldB = LAZY_LOGS ? ln(a.beta) - ln(b.beta) : a.lbeta - b.lbeta;
+    // one difference taken before the next pair of logarithms starts (registers)
+    if (LAZY_LOGS) asm volatile("" : "+v"(ldB));
     const double ldR = LAZY_LOGS ? ln(a.rho) - ln(b.rho) : a.lrho - b.lrho;
-    const double ldB = LAZY_LOGS ? ln(a.beta) - ln(b.beta) : a.lbeta - b.lbeta;
     const double dR = serR ? 1.0 : ldR;
     const double dB = serB ? 1.0 : db;
     const double q2 = rcp(dR * dB);
