@@ -386,7 +386,10 @@ __device__ __forceinline__ void vol_body(bool valid, int l, const double *Uq, co
   // almost every wave of the Taylor-Green state, 93 % of the vortex ensemble's), and
   // with two rows per lane (3D N = 3) the loops skip the per-pair branch test of the
   // log means (same bits).  With one row per lane the 3D kernels have no registers
-  // for it (spills; skipping the test at N = 4 measured 1.5 % slower).
+  // for it (spills; skipping the test at N = 4 measured 1.5 % slower).  In 2D a rough wave
+  // pays for the later logarithms where little work follows: the volume kernel at N = 1,
+  // K = 2,048, always taken / where needed: smooth 10.5 / 9.8 us, rough 10.4 / 11.0; N =
+  // 2: 12.1 / 11.4 and 12.0 / 12.7; the fused stage of these shapes is faster on both.
   constexpr bool SMOOTH_LOOPS = DIM == 3 && R > 1;
   constexpr bool LAZY = DIM == 2 || R > 1;   // face records
   constexpr bool LAZY_V = DIM == 2;          // volume records
@@ -1679,16 +1682,16 @@ template <class S> int vol_impl(const wadges_plan *p, int K, const double *vgeo,
     int rc = ensure_tables<S>(p, Drq, Dsq, Dtq, VqLq, VfPq, st, &tab);
     if (rc) return rc;
   }
-  constexpr int TPW = S::TPW;
-  static_assert(TPW >= 1, "Nq must fit in one wave");
-  const size_t smem = (size_t)TPW * VolSmem<S>::per_elem * sizeof(double);
-  const int blocks = (K + TPW - 1) / TPW;
   const double gm1 = p->gamma - 1.0;
   if constexpr (S::R > 1) {
     using X = Team<S>;
     team_vol_kernel<S><<<(K + X::E - 1) / X::E, X::T, X::bytes, st>>>(K, vgeo, vfgeo, nrJ, nsJ, ntJ, tab, Qf,
                                                               rhsQ, rhsQf, gm1, 1.0 / (2.0 * gm1));
   } else {
+    constexpr int TPW = S::TPW;
+    static_assert(TPW >= 1, "Nq must fit in one wave");
+    constexpr size_t smem = (size_t)TPW * VolSmem<S>::per_elem * sizeof(double);
+    const int blocks = (K + TPW - 1) / TPW;
     vol_kernel<S><<<blocks, WAVE, smem, st>>>(K, vgeo, vfgeo, nrJ, nsJ, ntJ, tab, Qf, rhsQ, rhsQf,
                                               gm1, 1.0 / (2.0 * gm1));
   }
@@ -1733,9 +1736,6 @@ template <class S> int stage_impl(const wadges_plan *p, int K, const double *vge
   const double *tab = nullptr;
   int rc = ensure_tables<S>(p, Drq, Dsq, Dtq, VqLq, VfPq, st, &tab);
   if (rc) return rc;
-  constexpr int TPW = S::TPW;
-  const size_t smem = (size_t)TPW * VolSmem<S>::per_elem * sizeof(double);
-  const int blocks = (K + TPW - 1) / TPW;
   const double g = p->gamma;
   StageArgs A{K,      vgeo,   vfgeo,   fgeo,   mapPq,  nrJ,     nsJ,  ntJ,
               tab,    VqLq,   VqPq,    VfPq,   Jq,     fa,      fb,   fdt,
@@ -1747,12 +1747,14 @@ template <class S> int stage_impl(const wadges_plan *p, int K, const double *vge
   } else {
     using Small = typename WideChoice<S>::Small;
     using Large = typename WideChoice<S>::Large;
+    constexpr int TPW = S::TPW;
+    constexpr size_t smem = (size_t)TPW * VolSmem<S>::per_elem * sizeof(double);
     if (K <= p->wide_k[0])
       stage_wide<Small><<<(K + Small::E - 1) / Small::E, Small::T, Small::bytes, st>>>(A);
     else if (K <= p->wide_k[1])
       stage_wide<Large><<<(K + Large::E - 1) / Large::E, Large::T, Large::bytes, st>>>(A);
     else
-      stage_kernel<S><<<blocks, WAVE, smem, st>>>(A);
+      stage_kernel<S><<<(K + TPW - 1) / TPW, WAVE, smem, st>>>(A);
   }
   return hip_check(hipGetLastError());
 }

@@ -11,10 +11,13 @@
 //     wave), so registers, not LDS, set the occupancy: three waves per SIMD;
 //   * a wave's walk is a quarter as long (3 + 12 steps instead of 12 + 48), so a
 //     small mesh finishes in a third of the time.
-// Fused stage, packed / this, microseconds on one card: K = 750 55.9 / 21.2; 2,058
-// 60.6 / 30.0; 6,000 89.6 / 61.3; 10,368 144 / 101; 24,576 245 / 229; 82,944 750 /
-// 741; 196,608 1,701 / 1,735 (there the packed kernel's fewer LDS reads weigh
-// more; its volume kernel 1,196 / 1,240, at 24,576 165 / 156).  The LDS is busy
+// Used for every mesh: faster than the packed kernels that give the same bits at every
+// size.  Fused stage, packed / this, microseconds on one card, launches back to back: K =
+// 750 56.5 / 21.2; 2,058 61.9 / 30.1; 6,000 91.2 / 61.4; 10,368 146 / 101; 24,576 248 /
+// 229; 82,944 793 / 754; 196,608 1,808 / 1,774.  Volume kernel: 24,576 190 / 179; 82,944
+// 533 / 493; 196,608 1,230 / 1,188.  (A packed kernel that sums straight through, without
+// the parts and so in other bits, takes 759 and 496 at 82,944, 1,742 and 1,158 at
+// 196,608, where its fewer LDS reads weigh more.)  The LDS is busy
 // 70 % of the time: a row's own record is read once per wave, the stride of an
 // element is LPE mod 32 doubles (3 % against a stride that makes the elements of a
 // wave meet in the banks), and neither records held in more registers (two waves per

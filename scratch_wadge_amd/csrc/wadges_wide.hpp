@@ -50,7 +50,7 @@ template <class S_, int E_, int W_, int CV_, int CF_> struct Wide {
 //   2D N = 4   K = 128    18.2 / 11.6   2,048  18.6 / 16.1    3,200  19.7 / 28.8
 //   2D N = 5   K = 512    26.5 / 16.9   1,058  27.1 / 30.3
 //   3D N = 1   K = 384    21.5 / 9.8    6,000  24.6 / 16.8   10,368  26.8 / 26.4
-//   3D N = 2   K = 162    25.3 / 11.2     750  25.6 / 13.4    1,296  26.2 / 24.0
+//   3D N = 2   K = 162    25.0 / 10.5     750  25.5 / 12.7    1,296  26.2 / 24.0
 //   3D N = 4   K = 384    47.3 / 36.0     750  49.1 / 45.1    1,296  67.8 / 83.9
 template <class S> struct WideChoice;
 template <> struct WideChoice<Shape<2, 3, 2>> {
